@@ -186,7 +186,9 @@ def _hc(g):
 
 
 def _captured(call):
-    """call() run once and then captured: (graph, the captured call's outputs)."""
+    """call() run once and then captured: (graph, the captured call's outputs).
+    Every buffer that call() names is kept by the caller's state, since the
+    graph holds bare addresses."""
     side = torch.cuda.Stream()
     side.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(side):
@@ -256,7 +258,8 @@ def prepare(case, seed):
             for l, (w, ws) in enumerate(s["w"])])
     elif kind == "expert":
         m, experts = s["layer"].meta, s["layer"].tensors["experts"]
-        ws = torch.empty(lib.expert_workspace_bytes(I), dtype=torch.uint8, device="cuda")
+        ws = s["ws"] = torch.empty(lib.expert_workspace_bytes(I), dtype=torch.uint8,
+                                   device="cuda")
         stride = m["expert_stride"]
 
         def call():
@@ -269,8 +272,9 @@ def prepare(case, seed):
         if case["tokens"] <= 8:
             s["graph"], s["out"] = _captured(lambda: _proj(lib, s["layers"]))
     elif kind == "ffn_step":
-        ws = torch.zeros(lib.ffn_step_workspace_bytes(s["layers"][0], MULT, case["tokens"]),
-                         dtype=torch.uint8, device="cuda")
+        ws = s["ws"] = torch.zeros(
+            lib.ffn_step_workspace_bytes(s["layers"][0], MULT, case["tokens"]),
+            dtype=torch.uint8, device="cuda")
 
         def call():
             s["state"].copy_(s["attended"])
@@ -279,7 +283,7 @@ def prepare(case, seed):
                     for state, layer, hc in zip(s["state"], s["layers"], s["hc"])]
         s["graph"], s["out"] = _captured(call)
     elif kind == "moe":
-        ws = lib.new_moe_workspace(s["layers"][0], case["tokens"], "cuda")
+        ws = s["ws"] = lib.new_moe_workspace(s["layers"][0], case["tokens"], "cuda")
         s["graph"], s["out"] = _captured(lambda: [
             lib.moe_forward(layer, x, s.get("ids"), workspace=ws, fast=case["fast"],
                             check=False) for layer, x in zip(s["layers"], s["x"])])
