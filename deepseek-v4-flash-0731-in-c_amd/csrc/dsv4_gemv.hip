@@ -969,8 +969,14 @@ __global__ __launch_bounds__(64) void k_bf16_rows_tiled(float *__restrict__ y,
 // The CLI's greedy token (src/cli/dsv4_run.c:357-359): best = 0, then every
 // v with logits[v] > logits[best] in order; so the first index of the
 // largest value, NaNs never taken, and 0 when logits[0] is NaN. One
-// workgroup per row: each thread keeps its first largest non-NaN value of
-// v = tid, tid + 256, ..., then (value, index) pairs merge with the larger
+// workgroup per row. Bound: one CU's load rate and latency (517 KB per row
+// at the model's vocabulary), so 16 waves with AM_Q 16-byte loads each in
+// flight: 147 us with 4 waves and one 4-byte load in flight each, about 8 us
+// now (one row of 129280). A thread's loads past the row are clamped to
+// the row's last 4 values (seen twice, which changes nothing). Each thread
+// keeps the first largest value of its ascending indices (bi < 0: none above
+// -inf; a row with no value above -inf gives 0, as the rule does whether
+// logits[0] is -inf or NaN), then (value, index) pairs merge with the larger
 // value, or the smaller index on equal values.
 __device__ __forceinline__ void am_merge(float &bv, int &bi, float ov, int oi) {
   if (oi >= 0 && (bi < 0 || ov > bv || (ov == bv && oi < bi))) {
@@ -979,20 +985,40 @@ __device__ __forceinline__ void am_merge(float &bv, int &bi, float ov, int oi) {
   }
 }
 
-__global__ __launch_bounds__(256) void k_argmax(int *idx, const float *logits, int vocab,
-                                                size_t stride) {
-  __shared__ float s_v[4];
-  __shared__ int s_i[4];
+#define AM_T 1024  // threads per row
+#define AM_Q 8     // 16-byte loads in flight per thread
+__global__ __launch_bounds__(AM_T) void k_argmax(int *idx, const float *logits, int vocab,
+                                                 size_t stride) {
+  __shared__ float s_v[AM_T / 64];
+  __shared__ int s_i[AM_T / 64];
   const int tid = threadIdx.x;
   const float *l = logits + (size_t)blockIdx.x * stride;
-  float bv = 0.0f;
+  float bv = -__builtin_inff();
   int bi = -1;
-  for (int v = tid; v < vocab; v += 256) {
-    const float f = l[v];
-    if (f == f && (bi < 0 || f > bv)) {
-      bv = f;
-      bi = v;
+  auto take = [&](float f, int i) {  // false for NaN
+    const bool t = f > bv;
+    bv = t ? f : bv;
+    bi = t ? i : bi;
+  };
+  if (vocab >= 4) {
+    for (long b = 0; b < vocab; b += 4 * AM_T * AM_Q) {
+      float4 f[AM_Q];
+      int at[AM_Q];
+#pragma unroll
+      for (int k = 0; k < AM_Q; ++k) {
+        at[k] = (int)min(b + 4 * (tid + AM_T * k), (long)vocab - 4);
+        __builtin_memcpy(&f[k], l + at[k], 16);  // rows may start at any float
+      }
+#pragma unroll
+      for (int k = 0; k < AM_Q; ++k) {
+        take(f[k].x, at[k]);
+        take(f[k].y, at[k] + 1);
+        take(f[k].z, at[k] + 2);
+        take(f[k].w, at[k] + 3);
+      }
     }
+  } else if (tid < vocab) {
+    take(l[tid], tid);
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1)
@@ -1003,7 +1029,7 @@ __global__ __launch_bounds__(256) void k_argmax(int *idx, const float *logits, i
   }
   __syncthreads();
   if (tid == 0) {
-    for (int w = 1; w < 4; ++w) am_merge(bv, bi, s_v[w], s_i[w]);
+    for (int w = 1; w < AM_T / 64; ++w) am_merge(bv, bi, s_v[w], s_i[w]);
     const float f0 = l[0];
     idx[blockIdx.x] = (f0 != f0 || bi < 0) ? 0 : bi;
   }
@@ -1418,7 +1444,7 @@ int dsv4g_argmax(int *idx, const float *logits, int vocab, int n, size_t stride,
                  void *stream) {
   if (!idx || !logits || vocab <= 0 || n <= 0 || stride < (size_t)vocab)
     return dsv4g_fail(DSV4G_EINVAL, "argmax: bad arguments");
-  hipLaunchKernelGGL(k_argmax, dim3((unsigned)n), dim3(256), 0, (hipStream_t)stream, idx,
+  hipLaunchKernelGGL(k_argmax, dim3((unsigned)n), dim3(AM_T), 0, (hipStream_t)stream, idx,
                      logits, vocab, stride);
   return dsv4g_check_launch("argmax");
 }

@@ -175,3 +175,23 @@ def test_expert_forward_shapes(env, hidden, inter):
                        inter, 10.0, gw)
     ref = orc.expert_forward(qx[0], qs[0], scales, weights, hidden, inter, 10, 0.618)
     assert same_bits(H(out), ref)
+
+
+@pytest.mark.parametrize("vocab", [1, 2, 3, 4, 5, 7, 4095, 4097, 32767, 32768, 32769, 32771,
+                                   129280])
+def test_greedy_row_lengths(env, vocab):
+    """Rows around the 4-value loads and the 32768-value rounds, rows that start
+    at any float (stride = an odd vocab), the maximum at the first, the last
+    and a clamped position, ties across the clamp, and rows of -inf and NaN."""
+    lib, torch = env["lib"], env["torch"]
+    rng = np.random.default_rng(vocab)
+    L = np.round(rng.standard_normal((7, vocab)) * 4).astype(np.float32)  # many ties
+    L[1, vocab - 1] = 99.0
+    L[2, 0] = 99.0
+    L[3, max(0, vocab - 3):] = 99.0
+    L[4, :] = -np.inf
+    L[5, :] = -np.inf
+    L[5, vocab // 2:] = np.nan
+    L[6, :] = np.nan
+    got = H(lib.argmax(torch.from_numpy(L).to(env["dev"])))
+    assert [int(g) for g in got] == [cli_greedy_fast(r) for r in L]
