@@ -4,6 +4,8 @@
 // router GEMV, the float-scale public GEMVs, dequantisers and the
 // synthetic-checkpoint quantisers.
 // The bit-exact GEMV row tiles are in dsv4_tiles.h.
+#include <algorithm>
+
 #include "dsv4_device.h"
 #include "dsv4_gpu_internal.h"
 #include "dsv4_tiles.h"
@@ -759,147 +761,151 @@ __global__ __launch_bounds__(256) void k_fp8_prodchain(float *__restrict__ y,
 
 // ================================================ batched BF16 rows ====
 // dsv4_gemv_bf16_batch / head_logits_batch (src/dsv4/dsv4_model.c:266-367,
-// 7371-7445) for many tokens, where the fp32 FMA issue rate, not HBM, is the
-// bound (64 tokens through the 129280 x 4096 head: 34 G dependent-chain
-// fmaf). Register blocking: lane = (row group rg = lane / 4, token group
-// tg = lane % 4) keeps 4 rows x KT tokens of chains, so each weight is read
-// and widened once for KT tokens and each x value read from LDS feeds 4 rows.
-// x moves through LDS in blocks of 8 columns (double-buffered, the next
-// block's weights and x in flight while the current block is chained); the
-// four token groups' rows sit 4 floats apart in LDS so that one 16-byte read
-// of all four hits distinct banks. Per (row, token) the fmaf chain runs in
-// column order, as the reference's. The reads of token k + 1 are issued
-// while token k is chained: an empty asm on token k's accumulators pins that
-// order, or the compiler hoists all reads of a block and runs out of
-// registers. in a multiple of 8, x 16-byte aligned; tokens [t0, t0 + 4 KT)
-// all present.
-template <int KT>
-__global__ __launch_bounds__(64) void k_bf16_rows_blocked(float *__restrict__ y,
-                                                          const float *__restrict__ x,
-                                                          const uint16_t *__restrict__ W, int in,
-                                                          int rows, int round_out, int t0) {
-  constexpr int NT = 4 * KT;            // tokens of this launch
-  constexpr int XS = NT * 8 + 16;       // one block: token t at 8 t + 4 (t / KT)
-  constexpr int NQ = (2 * NT + 63) / 64;  // 16-byte x pieces per lane per block
-  __shared__ __align__(16) float xs[2][XS];
-  const int lane = threadIdx.x, rg = lane >> 2, tg = lane & 3;
-  const int r0 = blockIdx.x * 64, rr = 4 * rg;
-  const int nrow = min(64, rows - r0);
+// 7371-7445) for 1 to 64 tokens on the fp32 matrix unit. v_mfma_f32_16x16x4
+// adds its four products to the accumulator one after another in k order,
+// each as one rounded fma with subnormals kept (test_f32_mfma_is_fma_chain
+// checks the bits), so a tile fed four columns at a time runs the reference's
+// column-order fmaf chain of each (row, token). Bound: the fp32 matrix rate,
+// 256 FLOP per clock and CU, twice the VALU's (64 tokens through the 129280 x
+// 4096 head are 34 G fma: 437 us at that rate, 540 us here, 1000 us as VALU chains; 16 tokens are
+// HBM-bound, 220 us against 700). Smaller matrices, whose VALU chains left
+// waves waiting, gain most: 16384 rows, 64 tokens 654 -> 90 us.
+//
+// A workgroup of 4 waves takes 64 MR rows, a wave 16 MR rows x 16 NT tokens
+// (MR NT accumulator tiles: four or more hide an MFMA's latency). Per step of
+// 64 columns a wave loads its rows coalesced (8 lanes per 128-byte piece, two
+// steps in flight), writes them to its own LDS rows (144 bytes apart:
+// conflict-free) and reads them back per (row, 8 columns); v_perm widens the
+// lane's column of each four. x is staged once per workgroup, the columns of a
+// step split by c % 4 so that one 16-byte read gives a lane its operand of
+// four MFMAs. A run's x tile is single-buffered: two workgroups share a CU, so
+// one computes while the other stages. The x loads of the next step are issued
+// ahead of the weights of the step after it (loads complete in order).
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+#define RM_XS 68  // LDS floats per token of an x tile: 64 + 4 (16 tokens: distinct banks)
+template <int NT, int MR>
+__global__ __launch_bounds__(256, 2) void k_bf16_rows_mfma(float *__restrict__ y,
+                                                           const float *__restrict__ x,
+                                                           const uint16_t *__restrict__ W,
+                                                           int in, int rows, int round_out,
+                                                           int t0, int nt) {
+  __shared__ __align__(16) float xs[16 * NT * RM_XS];
+  __shared__ __align__(16) uint4 tl[4][16 * MR * 9];
+  constexpr int LD = 2 * MR;  // 16-byte weight loads per lane and step
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, g = lane >> 4;
+  const int r0 = (blockIdx.x * 4 + wave) * 16 * MR;
+  const int nrow = __builtin_amdgcn_readfirstlane(max(0, min(16 * MR, rows - r0)));
   const uint32_t rb = 2u * (uint32_t)in;
   const BufRsrc rw = buf_rsrc(W + (size_t)r0 * in, (uint32_t)nrow * rb);
-  // rows past the tile's end read row 0 (in bounds) and are not stored
-  const uint32_t ro0 = rr < nrow ? (uint32_t)rr * rb : 0u;
-  const uint32_t ro1 = rr + 1 < nrow ? (uint32_t)(rr + 1) * rb : 0u;
-  const uint32_t ro2 = rr + 2 < nrow ? (uint32_t)(rr + 2) * rb : 0u;
-  const uint32_t ro3 = rr + 3 < nrow ? (uint32_t)(rr + 3) * rb : 0u;
-  const float *xb = x + (size_t)t0 * in;
-  // x staging: piece p = lane + 64 q (q < NQ <= 2) is token p / 2, columns
-  // 4 (p % 2) .. + 3; a lane past the last piece re-reads it and stores nothing
-  static_assert(NQ <= 2, "x staging holds two pieces per lane");
-  const int p0 = min(lane, 2 * NT - 1), p1 = min(lane + 64, 2 * NT - 1);
-  const float *xp0 = xb + (size_t)(p0 >> 1) * in + 4 * (p0 & 1);
-  const float *xp1 = xb + (size_t)(p1 >> 1) * in + 4 * (p1 & 1);
-  const int so0 = 4 * p0 + 4 * ((p0 >> 1) / KT);  // 8 t + 4 (p % 2) + 4 (t / KT)
-  const int so1 = 4 * p1 + 4 * ((p1 >> 1) / KT);
-  const bool st0 = lane < 2 * NT, st1 = NQ > 1 && lane + 64 < 2 * NT;
-  float acc[4][KT];
+  const BufRsrc rx = buf_rsrc(x + (size_t)t0 * in, (uint32_t)nt * 2u * rb);
+  const int lr = lane >> 3, lp = lane & 7;
+  const uint32_t lo = (uint32_t)lr * rb + 16u * lp;  // step t, rows 8 i + lr: + 8 rb i + 128 t
+  const int steps = in / 64;
+  // x staging: thread = (token tid / 4, 16 columns 16 (tid % 4) of the step);
+  // every load is issued without a branch, past the last step or token out of
+  // range (zeros, no access); tokens past the run are not stored
+  const uint32_t xo = (uint32_t)(tid >> 2) * 2u * rb + 64u * (uint32_t)(tid & 3);
+  float *xd = xs + (tid >> 2) * RM_XS + 4 * (tid & 3);
+  // bytes of the lane's column of four (two dwords) as a widened BF16
+  const uint32_t sel = 0x01000C0Cu + 0x02020000u * (uint32_t)g;
+  uint4 xr[4], T[2][LD];
 #pragma unroll
-  for (int j = 0; j < 4; ++j)
+  for (int j = 0; j < 4; ++j) xr[j] = buf_load16(rx, xo + 16u * j);
 #pragma unroll
-    for (int k = 0; k < KT; ++k) acc[j][k] = 0.0f;
-  uint4 w0 = buf_load16(rw, ro0), w1 = buf_load16(rw, ro1), w2 = buf_load16(rw, ro2),
-        w3 = buf_load16(rw, ro3);
-  float4 xr0 = *reinterpret_cast<const float4 *>(xp0), xr1 = xr0;
-  if (NQ > 1) xr1 = *reinterpret_cast<const float4 *>(xp1);
-  if (st0) *reinterpret_cast<float4 *>(&xs[0][so0]) = xr0;
-  if (st1) *reinterpret_cast<float4 *>(&xs[0][so1]) = xr1;
-  __syncthreads();
-  const int rd = 8 * KT * tg + 4 * tg;  // token KT tg of this lane's group
-  int b = 0;
-  for (int c0 = 0; c0 < in; c0 += 8) {
-    const bool more = c0 + 8 < in;
-    uint4 n0, n1, n2, n3;
-    if (more) {
-      const uint32_t o = 2u * (uint32_t)(c0 + 8);
-      n0 = buf_load16(rw, ro0 + o);
-      n1 = buf_load16(rw, ro1 + o);
-      n2 = buf_load16(rw, ro2 + o);
-      n3 = buf_load16(rw, ro3 + o);
-      xr0 = *reinterpret_cast<const float4 *>(xp0 + c0 + 8);
-      if (NQ > 1) xr1 = *reinterpret_cast<const float4 *>(xp1 + c0 + 8);
-    }
-    float wv[4][8];
-    const uint4 wq[4] = {w0, w1, w2, w3};
+  for (int d = 0; d < 2; ++d)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const uint32_t wd[4] = {wq[j].x, wq[j].y, wq[j].z, wq[j].w};
+    for (int i = 0; i < LD; ++i)
+      T[d][i] = buf_load16(rw, d < steps ? lo + 8u * rb * i + 128u * d : 0xFFFFFFF0u);
+  f32x4 acc[MR][NT];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        wv[j][2 * k] = u2f(wd[k] << 16);
-        wv[j][2 * k + 1] = u2f(wd[k] & 0xFFFF0000u);
+  for (int m = 0; m < MR; ++m)
+#pragma unroll
+    for (int n = 0; n < NT; ++n) acc[m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int tb = 0; tb < steps; tb += 2) {
+#pragma unroll
+    for (int d = 0; d < 2; ++d) {
+      const int t = tb + d;
+      __syncthreads();  // every wave is done with the last step's x
+      if (64 * NT == 256 || tid < 64 * NT) {
+        *reinterpret_cast<uint4 *>(xd) = make_uint4(xr[0].x, xr[1].x, xr[2].x, xr[3].x);
+        *reinterpret_cast<uint4 *>(xd + 16) = make_uint4(xr[0].y, xr[1].y, xr[2].y, xr[3].y);
+        *reinterpret_cast<uint4 *>(xd + 32) = make_uint4(xr[0].z, xr[1].z, xr[2].z, xr[3].z);
+        *reinterpret_cast<uint4 *>(xd + 48) = make_uint4(xr[0].w, xr[1].w, xr[2].w, xr[3].w);
+      }
+      const uint32_t xn = t + 1 < steps ? xo + 256u * (uint32_t)(t + 1) : 0xFFFFFF00u;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) xr[j] = buf_load16(rx, xn + 16u * j);
+#pragma unroll
+      for (int i = 0; i < LD; ++i) tl[wave][(8 * i + lr) * 9 + lp] = T[d][i];
+#pragma unroll
+      for (int i = 0; i < LD; ++i)
+        T[d][i] = buf_load16(rw, t + 2 < steps ? lo + 8u * rb * i + 128u * (t + 2) : 0xFFFFFFF0u);
+      __syncthreads();
+      if (t >= steps) break;  // uniform; an odd last step
+      // eight pieces of 8 columns: the reads of a piece are issued ahead of the
+      // MFMAs of the one before it (the empty asm keeps the compiler from
+      // hoisting every read of the step, which spilled)
+      f32x4 b[2][NT];
+      uint4 w[2][MR];
+      auto read = [&](int p) {
+        if (p % 2 == 0)
+#pragma unroll
+          for (int n = 0; n < NT; ++n)
+            b[p / 2 % 2][n] =
+                *reinterpret_cast<const f32x4 *>(xs + (16 * n + l16) * RM_XS + 16 * g + 2 * p);
+#pragma unroll
+        for (int m = 0; m < MR; ++m) w[p % 2][m] = tl[wave][(16 * m + l16) * 9 + p];
+      };
+      read(0);
+#pragma unroll
+      for (int p = 0; p < 8; ++p) {
+        asm volatile("" ::: "memory");
+        if (p + 1 < 8) read(p + 1);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int e = 0; e < 2; ++e)  // 4 columns
+#pragma unroll
+          for (int m = 0; m < MR; ++m) {
+            const uint4 wm = w[p % 2][m];
+            const float av = u2f(e ? __builtin_amdgcn_perm(wm.w, wm.z, sel)
+                                   : __builtin_amdgcn_perm(wm.y, wm.x, sel));
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+              acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                  av, b[p / 2 % 2][n][2 * (p % 2) + e], acc[m][n], 0, 0, 0);
+          }
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
-    const float *xl = &xs[b][rd];
-    float4 na = *reinterpret_cast<const float4 *>(xl);
-    float4 nb = *reinterpret_cast<const float4 *>(xl + 4);
-#pragma unroll
-    for (int k = 0; k < KT; ++k) {
-      const float4 xa = na, xc = nb;
-      if (k + 1 < KT) {
-        na = *reinterpret_cast<const float4 *>(xl + 8 * (k + 1));
-        nb = *reinterpret_cast<const float4 *>(xl + 8 * (k + 1) + 4);
-      }
-      asm volatile("" ::: "memory");
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        float a = acc[j][k];
-        a = fmaf(wv[j][0], xa.x, a);
-        a = fmaf(wv[j][1], xa.y, a);
-        a = fmaf(wv[j][2], xa.z, a);
-        a = fmaf(wv[j][3], xa.w, a);
-        a = fmaf(wv[j][4], xc.x, a);
-        a = fmaf(wv[j][5], xc.y, a);
-        a = fmaf(wv[j][6], xc.z, a);
-        a = fmaf(wv[j][7], xc.w, a);
-        acc[j][k] = a;
-      }
-      asm volatile("" : "+v"(acc[0][k]), "+v"(acc[1][k]), "+v"(acc[2][k]), "+v"(acc[3][k]));
-    }
-    if (more) {
-      if (st0) *reinterpret_cast<float4 *>(&xs[b ^ 1][so0]) = xr0;
-      if (st1) *reinterpret_cast<float4 *>(&xs[b ^ 1][so1]) = xr1;
-      w0 = n0;
-      w1 = n1;
-      w2 = n2;
-      w3 = n3;
-    }
-    __syncthreads();
-    b ^= 1;
   }
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int row = r0 + rr + j;
-    if (row < rows) {
+  for (int n = 0; n < NT; ++n) {
+    const int tok = 16 * n + l16;
+    if (tok >= nt) continue;
 #pragma unroll
-      for (int k = 0; k < KT; ++k) {
-        const float v = acc[j][k];
-        y[(size_t)(t0 + KT * tg + k) * rows + row] = round_out ? bf16_round(v) : v;
+    for (int m = 0; m < MR; ++m)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int row = 16 * m + 4 * g + v;
+        const float o = acc[m][n][v];
+        if (row < nrow) y[(size_t)(t0 + tok) * rows + r0 + row] = round_out ? bf16_round(o) : o;
       }
-    }
   }
 }
 
-// The same chains for 1 to 3 tokens (decode, and the remainder of a batch
-// split into runs of 4 KT), where HBM is the bound: a lane per output row
-// reading its own row would touch 64 cache lines per load, so the wave loads
-// tiles of 64 rows x 64 columns coalesced (lane l: rows 8 i + l / 8, 16
-// bytes at column 8 (l % 8)), writes them to LDS (rows 144 bytes apart, so
-// that the lanes' row reads hit distinct banks) and reads back its own row's
-// 64 columns. Two tiles are in flight while one is chained; x enters each
-// fmaf as a scalar operand. LDS holds one tile: the wave's LDS accesses run
-// in order, and the empty asms keep the compiler from moving them across
-// each other. in a multiple of 64; tokens [t0, t0 + TB) present.
+// The same chains for 1 or 2 tokens of a large matrix, where HBM is the bound: a
+// lane per output row reading its own row would touch 64 cache lines per load,
+// so the wave loads tiles of 64 rows x 64 columns coalesced (lane l: rows
+// 8 i + l / 8, 16 bytes at column 8 (l % 8)), writes them to LDS (rows 144
+// bytes apart, so that the lanes' row reads hit distinct banks) and reads back
+// its own row's 64 columns. Two tiles are in flight while one is chained; x
+// enters each fmaf as a scalar operand. LDS holds one tile: the wave's LDS
+// accesses run in order, and the empty asms keep the compiler from moving them
+// across each other. in a multiple of 64; tokens [t0, t0 + TB)
+// present. 129280 x 4096: 185 us, 2 tokens 223.
 #define RT_DEPTH 2
 template <int TB>
 __global__ __launch_bounds__(64) void k_bf16_rows_tiled(float *__restrict__ y,
@@ -1197,6 +1203,45 @@ static void launch_fp4_t(const GemvArgs *a, int nvec, int pair, hipStream_t st) 
   hipLaunchKernelGGL(k_gemv_fp4_t<NP>, grid, dim3(256), lds, st, *a, pair);
 }
 
+// Row tiles per wave (MR): the pick that leaves the busiest CU the fewest
+// tiles, ceil(workgroups / 256) * MR, and of equals the larger (x staged for
+// more rows) as long as it gives about two workgroups per CU, so that one
+// computes while the other stages. 129280 rows: MR 4, 505 workgroups (64
+// tokens 540 us, MR 1 565); 65536 rows: MR 1 (64 tokens 270 us, MR 4 with 256
+// workgroups 311); 98304 rows, 64 tokens: MR 2, 768 workgroups (393 us, MR 1
+// 406). Up to 16 tokens MR 2 is left out: the weight stream bounds, and more
+// waves keep more of it in flight (98304 rows: MR 1 155 us, MR 2 177).
+template <int NT>
+static void launch_rows_mfma_nt(float *y, const float *x, const uint16_t *W, int in, int out,
+                                int round_out, int t0, int n, hipStream_t st) {
+  int mr = 1;
+  long best = (out + 63L) / 64;
+  best = (best + 255) / 256;
+  for (int m = NT == 1 ? 4 : 2; m <= 4; m *= 2) {
+    const long wgs = (out + 64L * m - 1) / (64L * m), cost = (wgs + 255) / 256 * m;
+    if (wgs >= 500 && cost <= best) {
+      best = cost;
+      mr = m;
+    }
+  }
+  auto k = mr == 4 ? k_bf16_rows_mfma<NT, 4> : mr == 2 ? k_bf16_rows_mfma<NT, 2>
+                                                       : k_bf16_rows_mfma<NT, 1>;
+  hipLaunchKernelGGL(k, dim3((unsigned)((out + 64 * mr - 1) / (64 * mr))), dim3(256), 0, st, y, x,
+                     W, in, out, round_out, t0, n);
+}
+
+static void launch_rows_mfma(float *y, const float *x, const uint16_t *W, int in, int out,
+                             int round_out, int t0, int n, hipStream_t st) {
+  if (n <= 16)
+    launch_rows_mfma_nt<1>(y, x, W, in, out, round_out, t0, n, st);
+  else if (n <= 32)
+    launch_rows_mfma_nt<2>(y, x, W, in, out, round_out, t0, n, st);
+  else if (n <= 48)
+    launch_rows_mfma_nt<3>(y, x, W, in, out, round_out, t0, n, st);
+  else
+    launch_rows_mfma_nt<4>(y, x, W, in, out, round_out, t0, n, st);
+}
+
 extern "C" {
 
 int dsv4g_quant_fp8_act(float *qx, float *qscale, const float *x, int n, int nvec,
@@ -1393,21 +1438,23 @@ int dsv4g_gemv_bf16(float *y, const float *x, const uint16_t *W, int in, int out
   if (in <= 0 || out <= 0 || batch <= 0) return dsv4g_fail(DSV4G_EINVAL, "gemv_bf16: bad size");
   const size_t xb = (size_t)batch * in * 4;
   if (in % 64 == 0 && ((uintptr_t)x & 15) == 0 && (size_t)64 * in * 2 < 0xFFFF0000u) {
-    // runs of 64, 32, 16, 8 or 4 tokens through the register-blocked chains,
-    // a remainder of 1 to 3 through the tiled chains
-    const dim3 grid((out + 63) / 64);
+    // runs of up to 64 tokens through the matrix unit's chains; 1 or 2 tokens
+    // of a large matrix through the tiled chains (129280 rows: 1 token 185 us
+    // against 227, 2 tokens 223 against 230 to 250, but 3 tokens 245 against
+    // 240; one token of 110000 rows 186 against 176, of 65536 rows 143 against
+    // 107, of 16384 rows 95 against 39), and so do rows too wide for a run's x
+    // within one buffer range, two tokens at a time
+    const bool wide = (size_t)64 * in * 4 >= 0xFFFF0000u;
     for (int t0 = 0; t0 < batch;) {
-      const int rem = batch - t0;
-      const int tb = rem >= 64 ? 64 : rem >= 32 ? 32 : rem >= 16 ? 16 : rem >= 8 ? 8 : rem >= 4 ? 4
-                                                                                      : rem;
-      auto k = tb == 64 ? k_bf16_rows_blocked<16> : tb == 32 ? k_bf16_rows_blocked<8>
-               : tb == 16 ? k_bf16_rows_blocked<4> : tb == 8 ? k_bf16_rows_blocked<2>
-               : tb == 4 ? k_bf16_rows_blocked<1> : tb == 3 ? k_bf16_rows_tiled<3>
-               : tb == 2 ? k_bf16_rows_tiled<2> : k_bf16_rows_tiled<1>;
-      hipLaunchKernelGGL(k, grid, dim3(64), 0, (hipStream_t)stream, y, x, W, in, out, round_out,
-                         t0);
+      const int n = std::min(batch - t0, wide ? 2 : 64);
+      if (wide || (n <= 2 && out > 114688))
+        hipLaunchKernelGGL(n == 1 ? k_bf16_rows_tiled<1> : k_bf16_rows_tiled<2>,
+                           dim3((out + 63) / 64), dim3(64), 0, (hipStream_t)stream, y, x, W, in,
+                           out, round_out, t0);
+      else
+        launch_rows_mfma(y, x, W, in, out, round_out, t0, n, (hipStream_t)stream);
       DSV4G_TRY(dsv4g_check_launch("gemv_bf16"));
-      t0 += tb;
+      t0 += n;
     }
     return 0;
   }

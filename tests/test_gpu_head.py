@@ -108,9 +108,8 @@ def test_greedy_edges(env):
                                             (64, 2048, 40), (100, 1024, 20), (77, 4096, 3),
                                             (300, 1000, 3), (50, 2056, 9)])
 def test_bf16_batch_instances(env, rows, in_, batch):
-    """Every kernel form: for in a multiple of 64, the register-blocked chains
-    in runs of 64/32/16/8/4 tokens and the tiled chains for a remainder of 1
-    to 3 (5 = 4 + 1, 71 = 64 + 4 + 3, 40 = 32 + 8, ragged last row tiles);
+    """Every kernel form: for in a multiple of 64, the matrix unit's chains in
+    runs of up to 64 tokens (71 = 64 + 7, ragged token and row tiles);
     for other in, the x-in-LDS row chains (x up to 64 KB) and the
     one-row-per-(row, token) fallback."""
     orc, lib = env["orc"], env["lib"]
@@ -195,3 +194,53 @@ def test_greedy_row_lengths(env, vocab):
     L[6, :] = np.nan
     got = H(lib.argmax(torch.from_numpy(L).to(env["dev"])))
     assert [int(g) for g in got] == [cli_greedy_fast(r) for r in L]
+
+
+@pytest.mark.parametrize("kind", ["wide", "subnormal", "cancel"])
+def test_f32_mfma_is_fma_chain(env, kind):
+    """The batched rows run their chains on the fp32 matrix unit, four columns
+    an instruction: the same bits as the host's fmaf chain where every step
+    rounds (exponents over 2^-40..2^40), where terms and sums are subnormal,
+    and where the sum cancels."""
+    orc, lib = env["orc"], env["lib"]
+    rng = np.random.default_rng(17)
+    rows, in_, batch = 70, 192, 19
+    W = rng.standard_normal((rows, in_)).astype(np.float32)
+    x = rng.standard_normal((batch, in_)).astype(np.float32)
+    if kind == "wide":
+        W = np.ldexp(W, rng.integers(-20, 21, W.shape))
+        x = np.ldexp(x, rng.integers(-20, 21, x.shape))
+    elif kind == "subnormal":
+        W = np.ldexp(W, rng.integers(-80, -60, W.shape))
+        x = np.ldexp(x, rng.integers(-80, -60, x.shape))
+    else:
+        x[:, 1::2] = -x[:, ::2]
+        W[:, 1::2] = W[:, ::2]
+    W = bf16_bits(W.astype(np.float32))
+    x = x.astype(np.float32)
+    y = H(lib.gemv_bf16(T(env, x), T(env, W), in_, rows, 0))
+    for t in range(batch):
+        assert same_bits(y[t], orc.gemv_bf16(x[t], W, in_, rows, 0)), t
+
+
+@pytest.mark.parametrize("rows,batch", [(16384, 64), (32768 + 5, 4), (65537, 49), (129280, 17),
+                                        (129280, 48), (16384, 33), (130, 128), (1, 16),
+                                        (114688, 2), (114689, 2), (114689, 65), (114689, 66)])
+def test_bf16_batch_row_tiles(env, rows, batch):
+    """1, 2 and 4 row tiles per wave by the number of rows, 1 to 4 token tiles,
+    ragged in both, runs of 64, an odd number of 64-column steps: every token
+    equal to its one-token result, and the last row's to the host's chain.
+    Above 114688 rows 1 or 2 tokens take the tiled chains."""
+    orc, lib, torch, dev = env["orc"], env["lib"], env["torch"], env["dev"]
+    g = torch.Generator(device=dev)
+    g.manual_seed(rows + batch)
+    in_ = 192
+    W = (torch.randn(rows, in_, generator=g, device=dev) * 0.05).to(torch.bfloat16) \
+        .view(torch.int16).contiguous()
+    x = torch.randn(batch, in_, generator=g, device=dev)
+    y = lib.gemv_bf16(x, W, in_, rows, 0)
+    for t in range(batch):
+        one = lib.gemv_bf16(x[t:t + 1].contiguous(), W, in_, rows, 0)[0]
+        assert torch.equal(y[t].view(torch.int32), one.view(torch.int32)), t
+        last = orc.gemv_bf16(H(x[t]), H(W[-1:]).view(np.uint16), in_, 1, 0)
+        assert same_bits(H(y[t, -1:]), last), t
