@@ -772,25 +772,38 @@ __global__ __launch_bounds__(256) void k_fp8_prodchain(float *__restrict__ y,
 // waves waiting, gain most: 16384 rows, 64 tokens 654 -> 90 us.
 //
 // A workgroup of 4 waves takes 64 MR rows, a wave 16 MR rows x 16 NT tokens
-// (MR NT accumulator tiles: four or more hide an MFMA's latency). Per step of
-// 64 columns a wave loads its rows coalesced (8 lanes per 128-byte piece, two
-// steps in flight), writes them to its own LDS rows (144 bytes apart:
-// conflict-free) and reads them back per (row, 8 columns); v_perm widens the
-// lane's column of each four. x is staged once per workgroup, the columns of a
-// step split by c % 4 so that one 16-byte read gives a lane its operand of
-// four MFMAs. A run's x tile is single-buffered: two workgroups share a CU, so
-// one computes while the other stages. The x loads of the next step are issued
-// ahead of the weights of the step after it (loads complete in order).
+// (MR NT accumulator tiles: independent chains hide an MFMA's latency, 33
+// clocks back to back on one tile, 50 with an operand formed in between). Per
+// step of 64 columns a wave loads its rows coalesced (8 lanes per 128-byte
+// piece, D steps in flight) and writes them to its own LDS rows: one row tile
+// (WIDE) widened and split by c % 4, so that one 16-byte read is a lane's
+// operand of four MFMAs and nothing stands between them (router of 777 tokens
+// 63 -> 47 us); more row tiles as they are (144 bytes apart: conflict-free),
+// read back per (row, 8 columns), v_perm widening the lane's column of each
+// four, which the other tiles' MFMAs cover. x is staged once per workgroup,
+// split by c % 4 as well, double-buffered where 64 KB of LDS allow. The x
+// loads of a step are issued ahead of its weights (loads complete in order).
+//
+// ROUTER: the gate's rows; y is the scores sqrt(softplus(z)), choice the
+// scores plus the bias, and blockIdx.y the token tile.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 #define RM_XS 68  // LDS floats per token of an x tile: 64 + 4 (16 tokens: distinct banks)
-template <int NT, int MR>
+template <int NT, int MR, bool ROUTER>
 __global__ __launch_bounds__(256, 2) void k_bf16_rows_mfma(float *__restrict__ y,
                                                            const float *__restrict__ x,
                                                            const uint16_t *__restrict__ W,
                                                            int in, int rows, int round_out,
-                                                           int t0, int nt) {
-  __shared__ __align__(16) float xs[16 * NT * RM_XS];
-  __shared__ __align__(16) uint4 tl[4][16 * MR * 9];
+                                                           int t0, int nt, float *__restrict__ choice,
+                                                           const float *__restrict__ bias) {
+  if (ROUTER) {
+    t0 = blockIdx.y * 16 * NT;
+    nt = min(16 * NT, nt - t0);
+  }
+  constexpr int XB = NT * MR == 16 ? 1 : 2;  // x buffers (64 KB of LDS in all)
+  constexpr int D = NT * MR <= 2 ? 4 : 2;    // steps in flight
+  __shared__ __align__(16) float xs[XB][16 * NT * RM_XS];
+  constexpr bool WIDE = MR == 1;
+  __shared__ __align__(16) uint4 tl[4][16 * MR * (WIDE ? RM_XS / 4 : 9)];
   constexpr int LD = 2 * MR;  // 16-byte weight loads per lane and step
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -807,43 +820,54 @@ __global__ __launch_bounds__(256, 2) void k_bf16_rows_mfma(float *__restrict__ y
   // every load is issued without a branch, past the last step or token out of
   // range (zeros, no access); tokens past the run are not stored
   const uint32_t xo = (uint32_t)(tid >> 2) * 2u * rb + 64u * (uint32_t)(tid & 3);
-  float *xd = xs + (tid >> 2) * RM_XS + 4 * (tid & 3);
+  const int xd = (tid >> 2) * RM_XS + 4 * (tid & 3);
   // bytes of the lane's column of four (two dwords) as a widened BF16
   const uint32_t sel = 0x01000C0Cu + 0x02020000u * (uint32_t)g;
-  uint4 xr[4], T[2][LD];
+  uint4 xr[D][4], T[D][LD];
+  auto load = [&](int d, int t) {
+    const uint32_t xn = t < steps ? xo + 256u * (uint32_t)t : 0xFFFFFF00u;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) xr[j] = buf_load16(rx, xo + 16u * j);
-#pragma unroll
-  for (int d = 0; d < 2; ++d)
+    for (int j = 0; j < 4; ++j) xr[d][j] = buf_load16(rx, xn + 16u * j);
 #pragma unroll
     for (int i = 0; i < LD; ++i)
-      T[d][i] = buf_load16(rw, d < steps ? lo + 8u * rb * i + 128u * d : 0xFFFFFFF0u);
+      T[d][i] = buf_load16(rw, t < steps ? lo + 8u * rb * i + 128u * t : 0xFFFFFFF0u);
+  };
+#pragma unroll
+  for (int d = 0; d < D; ++d) load(d, d);
   f32x4 acc[MR][NT];
 #pragma unroll
   for (int m = 0; m < MR; ++m)
 #pragma unroll
     for (int n = 0; n < NT; ++n) acc[m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int tb = 0; tb < steps; tb += 2) {
+  for (int tb = 0; tb < steps; tb += D) {
 #pragma unroll
-    for (int d = 0; d < 2; ++d) {
+    for (int d = 0; d < D; ++d) {
       const int t = tb + d;
-      __syncthreads();  // every wave is done with the last step's x
+      if (XB == 1) __syncthreads();  // every wave is done with the last step's x
+      float *xw = xs[d % XB];
       if (64 * NT == 256 || tid < 64 * NT) {
-        *reinterpret_cast<uint4 *>(xd) = make_uint4(xr[0].x, xr[1].x, xr[2].x, xr[3].x);
-        *reinterpret_cast<uint4 *>(xd + 16) = make_uint4(xr[0].y, xr[1].y, xr[2].y, xr[3].y);
-        *reinterpret_cast<uint4 *>(xd + 32) = make_uint4(xr[0].z, xr[1].z, xr[2].z, xr[3].z);
-        *reinterpret_cast<uint4 *>(xd + 48) = make_uint4(xr[0].w, xr[1].w, xr[2].w, xr[3].w);
+        const uint4 *c = xr[d];
+        *reinterpret_cast<uint4 *>(xw + xd) = make_uint4(c[0].x, c[1].x, c[2].x, c[3].x);
+        *reinterpret_cast<uint4 *>(xw + xd + 16) = make_uint4(c[0].y, c[1].y, c[2].y, c[3].y);
+        *reinterpret_cast<uint4 *>(xw + xd + 32) = make_uint4(c[0].z, c[1].z, c[2].z, c[3].z);
+        *reinterpret_cast<uint4 *>(xw + xd + 48) = make_uint4(c[0].w, c[1].w, c[2].w, c[3].w);
       }
-      const uint32_t xn = t + 1 < steps ? xo + 256u * (uint32_t)(t + 1) : 0xFFFFFF00u;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) xr[j] = buf_load16(rx, xn + 16u * j);
-#pragma unroll
-      for (int i = 0; i < LD; ++i) tl[wave][(8 * i + lr) * 9 + lp] = T[d][i];
-#pragma unroll
-      for (int i = 0; i < LD; ++i)
-        T[d][i] = buf_load16(rw, t + 2 < steps ? lo + 8u * rb * i + 128u * (t + 2) : 0xFFFFFFF0u);
+      for (int i = 0; i < LD; ++i) {
+        const uint4 v = T[d][i];
+        if (WIDE) {
+          float2 *wd = reinterpret_cast<float2 *>(tl[wave]) + (8 * i + lr) * (RM_XS / 2) + lp;
+          wd[0] = make_float2(u2f(v.x << 16), u2f(v.z << 16));
+          wd[8] = make_float2(u2f(v.x & 0xFFFF0000u), u2f(v.z & 0xFFFF0000u));
+          wd[16] = make_float2(u2f(v.y << 16), u2f(v.w << 16));
+          wd[24] = make_float2(u2f(v.y & 0xFFFF0000u), u2f(v.w & 0xFFFF0000u));
+        } else {
+          tl[wave][(8 * i + lr) * 9 + lp] = v;
+        }
+      }
+      load(d, t + D);
       __syncthreads();
-      if (t >= steps) break;  // uniform; an odd last step
+      if (t >= steps) break;  // uniform; the last round may be short
       // eight pieces of 8 columns: the reads of a piece are issued ahead of the
       // MFMAs of the one before it (the empty asm keeps the compiler from
       // hoisting every read of the step, which spilled)
@@ -854,9 +878,14 @@ __global__ __launch_bounds__(256, 2) void k_bf16_rows_mfma(float *__restrict__ y
 #pragma unroll
           for (int n = 0; n < NT; ++n)
             b[p / 2 % 2][n] =
-                *reinterpret_cast<const f32x4 *>(xs + (16 * n + l16) * RM_XS + 16 * g + 2 * p);
+                *reinterpret_cast<const f32x4 *>(xw + (16 * n + l16) * RM_XS + 16 * g + 2 * p);
 #pragma unroll
-        for (int m = 0; m < MR; ++m) w[p % 2][m] = tl[wave][(16 * m + l16) * 9 + p];
+        for (int m = 0; m < MR; ++m) {
+          if (!WIDE)
+            w[p % 2][m] = tl[wave][(16 * m + l16) * 9 + p];
+          else if (p % 2 == 0)
+            w[p / 2 % 2][m] = tl[wave][(16 * m + l16) * (RM_XS / 4) + 4 * g + p / 2];
+        }
       };
       read(0);
 #pragma unroll
@@ -869,9 +898,10 @@ __global__ __launch_bounds__(256, 2) void k_bf16_rows_mfma(float *__restrict__ y
         for (int e = 0; e < 2; ++e)  // 4 columns
 #pragma unroll
           for (int m = 0; m < MR; ++m) {
-            const uint4 wm = w[p % 2][m];
-            const float av = u2f(e ? __builtin_amdgcn_perm(wm.w, wm.z, sel)
-                                   : __builtin_amdgcn_perm(wm.y, wm.x, sel));
+            const uint4 wm = w[WIDE ? p / 2 % 2 : p % 2][m];
+            const float av = u2f(WIDE ? p % 2 ? e ? wm.w : wm.z : e ? wm.y : wm.x
+                                 : e  ? __builtin_amdgcn_perm(wm.w, wm.z, sel)
+                                      : __builtin_amdgcn_perm(wm.y, wm.x, sel));
 #pragma unroll
             for (int n = 0; n < NT; ++n)
               acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(
@@ -891,7 +921,16 @@ __global__ __launch_bounds__(256, 2) void k_bf16_rows_mfma(float *__restrict__ y
       for (int v = 0; v < 4; ++v) {
         const int row = 16 * m + 4 * g + v;
         const float o = acc[m][n][v];
-        if (row < nrow) y[(size_t)(t0 + tok) * rows + r0 + row] = round_out ? bf16_round(o) : o;
+        const size_t at = (size_t)(t0 + tok) * rows + r0 + row;
+        if (row < nrow) {
+          if (ROUTER) {
+            const float sc = sqrt_softplus(o);
+            y[at] = sc;
+            choice[at] = sc + (bias ? bias[r0 + row] : 0.0f);
+          } else {
+            y[at] = round_out ? bf16_round(o) : o;
+          }
+        }
       }
   }
 }
@@ -1224,10 +1263,10 @@ static void launch_rows_mfma_nt(float *y, const float *x, const uint16_t *W, int
       mr = m;
     }
   }
-  auto k = mr == 4 ? k_bf16_rows_mfma<NT, 4> : mr == 2 ? k_bf16_rows_mfma<NT, 2>
-                                                       : k_bf16_rows_mfma<NT, 1>;
+  auto k = mr == 4 ? k_bf16_rows_mfma<NT, 4, false> : mr == 2 ? k_bf16_rows_mfma<NT, 2, false>
+                                                       : k_bf16_rows_mfma<NT, 1, false>;
   hipLaunchKernelGGL(k, dim3((unsigned)((out + 64 * mr - 1) / (64 * mr))), dim3(256), 0, st, y, x,
-                     W, in, out, round_out, t0, n);
+                     W, in, out, round_out, t0, n, nullptr, nullptr);
 }
 
 static void launch_rows_mfma(float *y, const float *x, const uint16_t *W, int in, int out,
@@ -1240,6 +1279,22 @@ static void launch_rows_mfma(float *y, const float *x, const uint16_t *W, int in
     launch_rows_mfma_nt<3>(y, x, W, in, out, round_out, t0, n, st);
   else
     launch_rows_mfma_nt<4>(y, x, W, in, out, round_out, t0, n, st);
+}
+
+// Every (token, expert) score and choice of the batched router, [T][E], exact.
+// Token tiles per wave: the fewest with at most one workgroup per CU (256
+// experts: 38 us up to 400 tokens, 47 at 777, 77 at 2048, 119 at 4096 beside
+// the shared expert's GEMMs).
+int dsv4g_launch_router_scores(float *score, float *choice, const float *x, const uint16_t *G,
+                               const float *bias, int T, int H, int E, hipStream_t st) {
+  const int egroups = (E + 63) / 64;
+  const long tiles = (T + 15L) / 16 * egroups;
+  const int nt = tiles <= 256 ? 1 : tiles <= 512 ? 2 : tiles <= 768 ? 3 : 4;
+  auto k = nt == 1 ? k_bf16_rows_mfma<1, 1, true> : nt == 2 ? k_bf16_rows_mfma<2, 1, true>
+         : nt == 3 ? k_bf16_rows_mfma<3, 1, true> : k_bf16_rows_mfma<4, 1, true>;
+  hipLaunchKernelGGL(k, dim3((unsigned)egroups, (unsigned)((T + 16 * nt - 1) / (16 * nt))),
+                     dim3(256), 0, st, score, x, G, H, E, 0, 0, T, choice, bias);
+  return dsv4g_check_launch("router_scores");
 }
 
 extern "C" {

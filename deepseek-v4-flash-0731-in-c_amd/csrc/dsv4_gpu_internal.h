@@ -42,6 +42,8 @@ int dsv4g_fail(int code, const char *fmt, ...);
 int dsv4g_check_launch(const char *what);
 int dsv4g_launch_gemv_fp4(const GemvArgs *a, int nvec, int nmat, void *stream);
 int dsv4g_launch_gemv_fp8(const GemvArgs *a, int nvec, int nmat, void *stream);
+int dsv4g_launch_router_scores(float *score, float *choice, const float *x, const uint16_t *G,
+                               const float *bias, int T, int H, int E, hipStream_t st);
 unsigned *dsv4g_decode_status_word(void *workspace);
 }
 

@@ -192,10 +192,10 @@ def test_batch_graph_replay_matches_eager(env):
 @pytest.mark.parametrize("hidden,inter,experts,n", [(1280, 384, 40, 100), (512, 256, 24, 300),
                                                     (2048, 640, 16, 257)])
 def test_batch_generic_widths(env, hidden, inter, experts, n):
-    """Widths off the model's (the per-window GEMM loops, the unsplit or
-    generic router logits), token counts on both sides of the few-token
-    router kernels (256) and not a multiple of the 64-token tile: routing
-    bit-exact, outputs within the tolerance, every token checked."""
+    """Widths off the model's (the per-window GEMM loops), token counts on both
+    sides of the few-token router kernel and of the folded shared expert (256)
+    and not a multiple of the 64-token tile: routing bit-exact, outputs within
+    the tolerance, every token checked."""
     orc, lib, dg = env["orc"], env["lib"], env["dg"]
     L = make_layer(orc, hidden, inter, experts, 4, seed=hidden + n, bias=True)
     L["bias"] = zipf_bias(experts, 3)
@@ -205,3 +205,31 @@ def test_batch_generic_widths(env, hidden, inter, experts, n):
     out, idx, wt = out.cpu().numpy(), idx.cpu().numpy(), wt.cpu().numpy()
     assert np.all(np.isfinite(out))
     check_batch(env, L, X, np.zeros(n, np.int32), out, idx, wt, range(n))
+
+
+@pytest.mark.parametrize("hidden,experts,n,topk,hash_vocab", [
+    (128, 5, 1, 2, 0), (384, 17, 15, 6, 0), (640, 320, 16, 6, 0), (4096, 256, 17, 6, 0),
+    (1280, 40, 170, 6, 0), (1280, 40, 171, 6, 7), (512, 24, 1024, 1, 0), (512, 24, 1025, 1, 0),
+    (384, 16, 600, 3, 5), (128, 5, 192, 2, 0), (128, 5, 193, 2, 0), (384, 320, 901, 6, 0),
+    (256, 320, 1700, 6, 0), (128, 320, 2500, 6, 0), (640, 70, 9000, 2, 0)])
+def test_batch_routing_exact(env, hidden, experts, n, topk, hash_vocab):
+    """The batched router (one lane per chain up to 192 tokens, beyond 16 x 16
+    tiles of chains on the fp32 matrix unit, 1 to 4 token tiles per wave) at
+    ragged token and expert tiles, both forms of the selection (1024 routes and
+    more), x not BF16-valued: every route and weight as the oracle's chains and
+    selection."""
+    orc, lib, dg = env["orc"], env["lib"], env["dg"]
+    L = make_layer(orc, hidden, 128, experts, topk, seed=hidden + n, bias=not hash_vocab,
+                   hash_vocab=hash_vocab)
+    DL = dg.DeviceLayer.from_host(L, env["dev"])
+    rng = np.random.default_rng(n)
+    X = rng.standard_normal((n, hidden)).astype(np.float32)
+    tok = (np.arange(n) % max(hash_vocab, 1)).astype(np.int32)
+    _, idx, wt = lib.moe_forward_batch(DL, T(env, X), T(env, tok))
+    idx, wt = idx.cpu().numpy(), wt.cpu().numpy()
+    for t in range(0, n, max(1, n // 64)):
+        z = orc.gemv_bf16(X[t], L["gate_w"], hidden, experts, 0)
+        row = L["tid2eid"][tok[t]] if hash_vocab else None
+        i, w = orc.route(z, L["bias"], row, topk, 1.5)
+        assert np.array_equal(idx[t], i), t
+        assert same_bits(wt[t], w), t
