@@ -247,6 +247,69 @@ __device__ __forceinline__ void hc_store_chunk(const float4 *v, const HcLane<PER
   if ((threadIdx.x & 63) == 0) st_flag_relaxed(flag, c + 1);
 }
 
+// The scale of token t from its sum of squares est (any order), the mixes
+// times it, and the split (one wave).
+__device__ __forceinline__ void hc_scale_split(const HcArgs &a, const float *state, int t,
+                                               double est, float *s_mix, float *s_pre,
+                                               float *s_post, float *s_comb) {
+  const int lane = threadIdx.x & 63, m = a.mult, K = m * a.hid, mix_n = (2 + m) * m;
+  bool exact;
+  float rs = rms_scale_bounded(est, K, a.rms_eps, &exact);
+  if (!exact) {  // every lane repeats the sum in index order
+    double ss = 0.0;
+    for (int i = 0; i < K; i++) {
+      const double d = (double)state[i];
+      ss += d * d;
+    }
+    rs = rms_scale(ss, K, a.rms_eps);
+  }
+  if (lane < mix_n) s_mix[lane] = s_mix[lane] * rs;
+  __builtin_amdgcn_wave_barrier();
+  hc_split_wave(s_pre, s_post, s_comb, s_mix, a.scale3, a.base, m, a.iters, a.hc_eps);
+  if (lane < m) a.post[(size_t)t * m + lane] = s_post[lane];
+  if (lane < m * m) a.comb[(size_t)t * m * m + lane] = s_comb[lane];
+}
+
+// bin = bf16(sum_i pre[i] * state[i][c]), then the optional RMSNorm (the whole
+// workgroup, s_pre visible to it).
+__device__ __forceinline__ void hc_bin_norm(const HcArgs &a, const float *state, int t,
+                                            const float *s_pre, double *s_part, float *s_scale,
+                                            float *s_bin) {
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, m = a.mult, hid = a.hid;
+  double ss = 0.0;
+  for (int c = tid; c < hid; c += blockDim.x) {
+    float acc = 0.0f;
+    for (int i = 0; i < m; i++) acc = fmaf(s_pre[i], state[(size_t)i * hid + c], acc);
+    const float b = bf16_round(acc);
+    s_bin[c] = b;
+    ss += (double)b * (double)b;
+  }
+  float *out = a.bin + (size_t)t * hid;
+  if (!a.norm_w) {
+    for (int c = tid; c < hid; c += blockDim.x) out[c] = s_bin[c];
+    return;
+  }
+  ss = wave_sum_d(ss);
+  if (lane == 0) s_part[wave] = ss;
+  __syncthreads();
+  if (tid == 0) {
+    double est = 0.0;
+    for (int w = 0; w < (int)(blockDim.x >> 6); w++) est += s_part[w];
+    bool exact;
+    float r = rms_scale_bounded(est, hid, a.rms_eps, &exact);
+    if (!exact) {
+      double s2 = 0.0;
+      for (int c = 0; c < hid; c++) s2 += (double)s_bin[c] * (double)s_bin[c];
+      r = rms_scale(s2, hid, a.rms_eps);
+    }
+    *s_scale = r;
+  }
+  __syncthreads();
+  const float r = *s_scale;
+  for (int c = tid; c < hid; c += blockDim.x)
+    out[c] = bf16_round(s_bin[c] * r * bf16_to_f32(a.norm_w[c]));
+}
+
 // One workgroup of NW waves (4 or 8) per token. The waves of a workgroup sit
 // on the CU's four SIMDs in turn (wave w on SIMD w % 4), and the chain wave
 // issues an instruction for every step of its 24 chains, so SIMD 0 is left
@@ -357,65 +420,259 @@ __global__ void __launch_bounds__(64 * NW) k_hc_pre(HcArgs a) {
   __syncthreads();
 
   // ---- hc_pre's scale, the mixes and the split (wave 0)
-  if (wave == 0) {
-    if (lane == 0) {
-      const double est = s_part[0];
-      bool exact;
-      float rs = rms_scale_bounded(est, K, a.rms_eps, &exact);
-      if (!exact) {
-        double ss = 0.0;
-        for (int i = 0; i < K; i++) {
-          const double d = (double)state[i];
-          ss += d * d;
-        }
-        rs = rms_scale(ss, K, a.rms_eps);
-      }
-      s_scale = rs;
+  if (wave == 0) hc_scale_split(a, state, t, s_part[0], s_mix, s_pre, s_post, s_comb);
+  __syncthreads();
+  // ---- bin (over the ring, free now), then the optional RMSNorm
+  hc_bin_norm(a, state, t, s_pre, s_part, &s_scale, lds);
+}
+
+// ---- few tokens: the chains split.
+// A chain acc = fmaf(w, x, acc) moves on the grid of acc's binade: as long as
+// every result stays in its binade, a start shifted by d gives every result
+// shifted by d, exactly, if d is a multiple of twice the coarsest grid met
+// (then also ties round alike). So the chain of a mix is cut into SEG
+// segments that run at the same time from guesses (the prefix of the products
+// in double, rounded): 8 candidates per segment, the floats base | j around
+// the guess, cover the residues of 8 grid steps, and the true start a then
+// gives the true end r_j + (a - (base | j)) for j = a's low bits, provided
+// |a - (base | j)| is below the smallest distance of the candidate's results
+// from a binade's ends, and no result lies more than two binades above the
+// start (8 grid steps there = 2 of the coarsest). Where that does not hold the
+// segment is run again from its true start, so the result is always the
+// chain's, bit for bit; a start equal to a candidate needs no condition.
+//  - Boundaries: each the multiple of 16 columns with the largest |prefix| of
+//    its 128 columns (a small start has a fine grid, which later results
+//    leave: without the choice 3.6 segments of 128 per chain miss, with it
+//    0.45, by simulation on normal products).
+//  - A lane runs 4 candidates of one segment (256 lanes); the margins are kept
+//    for its first one and widened by the spread to its last (rounding is
+//    monotone: the others lie between).
+//  - Eight segments compose to one the same way (128 lanes, all 8 candidates
+//    of 16 such), so the serial walk has 16 steps; one whose conditions fail is
+//    walked segment by segment.
+// A workgroup per mix and token: 24 CUs share what one wave of one CU did (83
+// us for one token; its chain of 16384 dependent fmaf runs at 10.5 clocks a
+// step). Bound now: launch, one round trip of the row and the state (128 KB
+// per workgroup), then instruction issue of the 4 chain waves. The mix goes to
+// bin's row of the token, where k_hc_finish reads it.
+constexpr int SP_T = 1024;         // threads, and 16-column pieces at most
+constexpr int SP_SEG = 128;        // segments: 8 pieces each (fewer for a shorter row)
+constexpr int SP_MAXK = 16 * SP_T;
+constexpr int SP_MINK = 2048;
+constexpr int SP_REC = 13;         // dwords per record: r[8], base, margin[2], top, pad (odd)
+constexpr int SP_SREC = 17;        // per eight segments: end[8], margin[8], pad (odd)
+
+__host__ __device__ constexpr int sp_at(int c) { return c + 4 * (c >> 6); }  // LDS column
+constexpr size_t sp_lds(int K) {
+  return ((size_t)2 * sp_at(K) + SP_SEG * SP_REC + SP_SEG / 8 * SP_SREC + 2 * SP_SEG) * 4;
+}
+
+// acc over columns [c, e) (multiples of 16), in order.
+__device__ __forceinline__ float sp_chain(const float *w, const float *x, int c, int e,
+                                          float acc) {
+  for (; c < e; c += 16) {
+    const float4 *wp = (const float4 *)(w + sp_at(c)), *xp = (const float4 *)(x + sp_at(c));
+    float4 wv[4], xv[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      wv[q] = wp[q];
+      xv[q] = xp[q];
     }
-    __builtin_amdgcn_wave_barrier();
-    const float rs = s_scale;
-    if (lane < mix_n) s_mix[lane] = s_mix[lane] * rs;
-    __builtin_amdgcn_wave_barrier();
-    hc_split_wave(s_pre, s_post, s_comb, s_mix, a.scale3, a.base, m, a.iters, a.hc_eps);
-    if (lane < m) a.post[(size_t)t * m + lane] = s_post[lane];
-    if (lane < m * m) a.comb[(size_t)t * m * m + lane] = s_comb[lane];
+    fma_group(acc, wv, xv);
+  }
+  return acc;
+}
+
+// A start a (bits A) against a record's candidate j of base b with end r and
+// margin m: true, the end and what is left of the margin, if the end follows.
+__device__ __forceinline__ bool sp_step(float a, uint32_t b, float r, float m, float *end,
+                                        float *left) {
+  const uint32_t A = __float_as_uint(a);
+  const float d = a - __uint_as_float(b | (A & 7u));
+  *end = d == 0.0f ? r : r + d;
+  *left = m - fabsf(d) * 1.0001f;
+  return (A >> 23) == (b >> 23) && (d == 0.0f || fabsf(d) < m);
+}
+
+__global__ void __launch_bounds__(SP_T) k_hc_mix_split(float *__restrict__ bin,
+                                                       const float *__restrict__ state,
+                                                       const float *__restrict__ fn, int K,
+                                                       int mix_n, int hid) {
+  extern __shared__ __align__(16) float lds[];
+  __shared__ double s_wave[SP_T / 64];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int mix = blockIdx.x, t = blockIdx.y;
+  float *lw = lds, *lx = lds + sp_at(K);
+  float *rec = lx + sp_at(K), *srec = rec + SP_SEG * SP_REC;
+  int *beg = (int *)(srec + SP_SEG / 8 * SP_SREC);  // first column of each segment
+  const int np = K / 16, nseg = (np + 7) / 8;       // K % 16 == 0
+
+  // ---- the row and the state into LDS; thread = one 16-column piece, whose
+  // sum of products and prefix are formed in double
+  double sum = 0.0;
+  if (tid < np) {
+    const float4 *wp = (const float4 *)(fn + (size_t)mix * K + 16 * tid);
+    const float4 *xp = (const float4 *)(state + (size_t)t * K + 16 * tid);
+    float4 wv[4], xv[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      wv[q] = wp[q];
+      xv[q] = xp[q];
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      ((float4 *)(lw + sp_at(16 * tid)))[q] = wv[q];
+      ((float4 *)(lx + sp_at(16 * tid)))[q] = xv[q];
+      sum += (double)wv[q].x * xv[q].x + (double)wv[q].y * xv[q].y + (double)wv[q].z * xv[q].z +
+             (double)wv[q].w * xv[q].w;
+    }
+  }
+  double inc = sum;  // inclusive over the wave
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const double v = __shfl_up(inc, o);
+    if (lane >= o) inc += v;
+  }
+  if (lane == 63) s_wave[wave] = inc;
+  __syncthreads();
+  double pre = inc - sum;
+  for (int w = 0; w < wave; w++) pre += s_wave[w];
+  // ---- boundaries and guesses: segment s starts at one of the pieces 8 s ..
+  // 8 s + 7, segment 0 at column 0 from the chain's own start
+  {
+    const float g = (float)pre;
+    float m = tid < np ? (g == g ? fabsf(g) : 0.0f) : -1.0f;
+    int p = tid;
+#pragma unroll
+    for (int o = 1; o < 8; o <<= 1) {
+      const float om = __shfl_xor(m, o);
+      const int op = __shfl_xor(p, o);
+      if (om > m || (om == m && op < p)) {
+        m = om;
+        p = op;
+      }
+    }
+    if (tid < 8) p = 0;
+    if (tid == p) {
+      beg[tid / 8] = 16 * tid;
+      rec[tid / 8 * SP_REC + 8] = tid == 0 ? 0.0f : __uint_as_float(__float_as_uint(g) & ~7u);
+    }
   }
   __syncthreads();
-
-  // ---- bin = bf16(sum_i pre[i] * state[i][c]), then the optional RMSNorm
-  float *s_bin = lds;  // the ring is free now
-  double ss = 0.0;
-  for (int c = tid; c < hid; c += blockDim.x) {
-    float acc = 0.0f;
-    for (int i = 0; i < m; i++) acc = fmaf(s_pre[i], state[(size_t)i * hid + c], acc);
-    const float b = bf16_round(acc);
-    s_bin[c] = b;
-    ss += (double)b * (double)b;
+  // ---- the segments: lane = (segment tid / 2, candidates 4 (tid % 2) .. + 3)
+  if (tid < 2 * nseg) {
+    const int s = tid >> 1, h = tid & 1, end = s + 1 < nseg ? beg[s + 1] : K;
+    const uint32_t base = __float_as_uint(rec[s * SP_REC + 8]);
+    float r[4], mgn = __builtin_inff(), top = 0.0f, spread = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 4; j++) r[j] = __uint_as_float(base | (4 * h + j));
+    for (int c = beg[s]; c < end; c += 16) {
+      const float4 *wp = (const float4 *)(lw + sp_at(c)), *xp = (const float4 *)(lx + sp_at(c));
+      float4 wv[4], xv[4];
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        wv[q] = wp[q];
+        xv[q] = xp[q];
+      }
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const float ws[4] = {wv[q].x, wv[q].y, wv[q].z, wv[q].w};
+        const float xs[4] = {xv[q].x, xv[q].y, xv[q].z, xv[q].w};
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+#pragma unroll
+          for (int j = 0; j < 4; j++) r[j] = fmaf(ws[i], xs[i], r[j]);
+          // distances to the binade's lower and upper end
+          const float p = __uint_as_float(__float_as_uint(r[0]) & 0xFF800000u);
+          const float lo = r[0] - p, hi = p - lo;
+          mgn = fminf(mgn, fminf(fabsf(lo), fabsf(hi)));
+          top = fmaxf(top, fabsf(r[0]));
+          spread = fmaxf(spread, fabsf(r[3] - r[0]));
+        }
+      }
+    }
+    // no result more than two binades above the start, else no shift at all
+    const bool grid = (__float_as_uint(top) >> 23) <= ((base >> 23) & 255u) + 2u;
+    const float m = mgn * 0.999f - spread * 1.001f;
+    float *R = rec + s * SP_REC;
+#pragma unroll
+    for (int j = 0; j < 4; j++) R[4 * h + j] = r[j];
+    R[9 + h] = grid && m > 0.0f ? m : 0.0f;
+    if (h == 0) R[11] = top;
   }
-  float *out = a.bin + (size_t)t * hid;
-  if (!a.norm_w) {
-    for (int c = tid; c < hid; c += blockDim.x) out[c] = s_bin[c];
-    return;
+  __syncthreads();
+  // ---- eight segments at a time: lane = (group tid / 8, candidate tid % 8)
+  const int ngrp = (nseg + 7) / 8;
+  if (tid < 8 * ngrp) {
+    const int q = tid >> 3, s1 = min(8 * q + 8, nseg);
+    const uint32_t base = __float_as_uint(rec[8 * q * SP_REC + 8]);
+    float a = __uint_as_float(base | (tid & 7)), m = __builtin_inff(), top = 0.0f;
+    bool ok = true;
+    for (int s = 8 * q; s < s1; s++) {
+      const float *R = rec + s * SP_REC;
+      const int j = __float_as_uint(a) & 7;
+      float end, left;
+      ok = sp_step(a, __float_as_uint(R[8]), R[j], R[9 + (j >> 2)], &end, &left) && ok;
+      a = end;
+      m = fminf(m, left);
+      top = fmaxf(top, R[11]);
+    }
+    const bool grid = (__float_as_uint(top) >> 23) <= ((base >> 23) & 255u) + 2u;
+    srec[q * SP_SREC + (tid & 7)] = a;
+    srec[q * SP_SREC + 8 + (tid & 7)] = !ok ? -1.0f : grid && m > 0.0f ? m : 0.0f;
+  }
+  __syncthreads();
+  // ---- the walk (one wave, every lane the same)
+  if (wave != 0) return;
+  float a = 0.0f;
+  for (int q = 0; q < ngrp; q++) {
+    const int j = __float_as_uint(a) & 7;
+    const float m = srec[q * SP_SREC + 8 + j];
+    float end, left;
+    if (sp_step(a, __float_as_uint(rec[8 * q * SP_REC + 8]), srec[q * SP_SREC + j], m, &end,
+                &left) && m >= 0.0f) {
+      a = end;
+      continue;
+    }
+    for (int s = 8 * q; s < min(8 * q + 8, nseg); s++) {
+      const float *R = rec + s * SP_REC;
+      const int js = __float_as_uint(a) & 7;
+      if (sp_step(a, __float_as_uint(R[8]), R[js], R[9 + (js >> 2)], &end, &left))
+        a = end;
+      else
+        a = sp_chain(lw, lx, beg[s], s + 1 < nseg ? beg[s + 1] : K, a);
+    }
+  }
+  if (lane == 0) bin[(size_t)t * hid + mix] = a;
+}
+
+// What follows the mixes (in bin's row): hc_pre's scale, the split, bin and
+// the optional RMSNorm, one workgroup per token.
+constexpr int HF_T = 512;
+__global__ void __launch_bounds__(HF_T) k_hc_finish(HcArgs a) {
+  extern __shared__ __align__(16) float lds[];
+  __shared__ float s_mix[64], s_pre[8], s_post[8], s_comb[64], s_scale;
+  __shared__ double s_part[HF_T / 64];
+  const int t = blockIdx.x, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int m = a.mult, hid = a.hid, K = m * hid, mix_n = (2 + m) * m;
+  const float *state = a.state + (size_t)t * K;
+  if (tid < mix_n) s_mix[tid] = a.bin[(size_t)t * hid + tid];
+  double ss = 0.0;
+  for (int i = 4 * tid; i < K; i += 4 * HF_T) {
+    const float4 x = *(const float4 *)(state + i);
+    const double x0 = x.x, x1 = x.y, x2 = x.z, x3 = x.w;
+    ss += x0 * x0 + x1 * x1 + x2 * x2 + x3 * x3;
   }
   ss = wave_sum_d(ss);
   if (lane == 0) s_part[wave] = ss;
   __syncthreads();
-  if (tid == 0) {
+  if (wave == 0) {
     double est = 0.0;
-    for (int w = 0; w < (int)(blockDim.x >> 6); w++) est += s_part[w];
-    bool exact;
-    float r = rms_scale_bounded(est, hid, a.rms_eps, &exact);
-    if (!exact) {
-      double s2 = 0.0;
-      for (int c = 0; c < hid; c++) s2 += (double)s_bin[c] * (double)s_bin[c];
-      r = rms_scale(s2, hid, a.rms_eps);
-    }
-    s_scale = r;
+    for (int w = 0; w < HF_T / 64; w++) est += s_part[w];
+    hc_scale_split(a, state, t, est, s_mix, s_pre, s_post, s_comb);
   }
   __syncthreads();
-  const float r = s_scale;
-  for (int c = tid; c < hid; c += blockDim.x)
-    out[c] = bf16_round(s_bin[c] * r * bf16_to_f32(a.norm_w[c]));
+  hc_bin_norm(a, state, t, s_pre, s_part, &s_scale, lds);
 }
 
 // rmsnorm_bf16 over rows of x (one workgroup per row); y may alias x.
@@ -492,6 +749,13 @@ int hc_ring(int mult) {
 
 bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 
+bool overlap(const float *a, size_t na, const float *b, size_t nb) {
+  return (uintptr_t)a < (uintptr_t)(b + nb) && (uintptr_t)b < (uintptr_t)(a + na);
+}
+
+// Up to this many tokens hc_pre's chains are split over a workgroup per mix.
+constexpr int HC_SPLIT_TOKENS = 40;
+
 }  // namespace
 
 extern "C" {
@@ -545,6 +809,22 @@ int dsv4g_hc_pre(float *bin, float *post, float *comb, const float *state, const
   a.ring = hc_ring(mult);
   a.rms_eps = rms_eps;
   a.hc_eps = hc_eps;
+  const int K = mult * hidden, mix_n = (2 + mult) * mult;
+  if (n_tokens <= HC_SPLIT_TOKENS && K % 16 == 0 && K >= SP_MINK && K <= SP_MAXK &&
+      mix_n <= hidden && !overlap(bin, (size_t)n_tokens * hidden, state, (size_t)n_tokens * K) &&
+      !overlap(bin, (size_t)n_tokens * hidden, fn, (size_t)mix_n * K) &&
+      !overlap(bin, (size_t)n_tokens * hidden, scale3, 3) &&
+      !overlap(bin, (size_t)n_tokens * hidden, base, mix_n)) {
+    // more than the default 64 KB of LDS (a host-side setting of the kernel)
+    DSV4G_HIP(hipFuncSetAttribute((const void *)k_hc_mix_split,
+                                  hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)sp_lds(SP_MAXK)));
+    hipLaunchKernelGGL(k_hc_mix_split, dim3(mix_n, n_tokens), dim3(SP_T), sp_lds(K),
+                       (hipStream_t)stream, bin, state, fn, K, mix_n, hidden);
+    hipLaunchKernelGGL(k_hc_finish, dim3(n_tokens), dim3(HF_T), (size_t)hidden * sizeof(float),
+                       (hipStream_t)stream, a);
+    return dsv4g_check_launch("hc_pre");
+  }
   const size_t ring = (size_t)a.ring * ((2 + mult) * mult + 1) * HC_RS * sizeof(float);
   const size_t lds = std::max(ring, (size_t)hidden * sizeof(float));
   if (lds > HC_LDS_BUDGET)

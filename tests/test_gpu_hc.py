@@ -251,3 +251,78 @@ def test_ffn_step_full_size(env):
     lib.check_decode_status(ws)
     print(f"\nhc_pre+norm {t_pre:.1f} us, hc_post {t_post:.1f} us, ffn_step {t_step:.1f} us "
           f"(1 token, host-timed launches)", flush=True)
+
+
+@pytest.mark.parametrize("mult,hid,n", [(4, 4096, 1), (4, 4096, 40), (4, 4096, 41), (1, 2048, 2),
+                                        (1, 16384, 1), (2, 1032, 1), (4, 516, 3), (7, 304, 2),
+                                        (3, 5456, 1), (4, 508, 1)])
+def test_hc_pre_split_chains(env, mult, hid, n):
+    """The chains split over segments (rows of 2048 to 16384 columns, 16 to 63
+    mixes, ragged last segments, up to 40 tokens) and the shapes just outside."""
+    orc, lib = env["orc"], env["lib"]
+    rng = np.random.default_rng(mult * 1000 + hid + n)
+    _, fn, sc, base = hc_inputs(rng, mult, hid)
+    S = bf16_values(rng.standard_normal((n, mult * hid)).astype(np.float32))
+    norm = bf16_bits((1.0 + 0.1 * rng.standard_normal(hid)).astype(np.float32))
+    b, p, c = (H(v) for v in lib.hc_pre(T(env, S), T(env, fn), T(env, sc), T(env, base), mult,
+                                        T(env, norm)))
+    for t in range(0, n, max(1, n // 8)):
+        ob, op, oc = orc.hc_pre(S[t], fn, sc, base, mult)
+        assert same_bits(p[t], op) and same_bits(c[t], oc), t
+        assert same_bits(b[t], orc.rmsnorm_bf16(ob[None], norm, 1e-6, 1)[0]), t
+
+
+@pytest.mark.parametrize("kind", ["zeros", "growing", "ones", "cancelling", "power_of_two",
+                                  "tiny", "subnormal", "huge", "steps", "zero_crossings", "sparse"])
+def test_hc_pre_split_chain_values(env, kind):
+    """Sums whose segments do not follow from their guesses: exact zeros, sums
+    that double from segment to segment, ties at every step, sums that return
+    to zero, that stay at a power of two, subnormal and overflowing sums. The
+    mixes reach the outputs through post and comb (scale 1, base 0)."""
+    orc, lib = env["orc"], env["lib"]
+    mult, hid = 4, 4096
+    K, mix_n = mult * hid, 24
+    rng = np.random.default_rng(5)
+    _, fn, sc, base = hc_inputs(rng, mult, hid)
+    S = bf16_values(rng.standard_normal(K).astype(np.float32))
+    k = np.arange(K)
+    if kind == "zeros":
+        S[:] = 0
+    elif kind == "growing":
+        S = bf16_values(np.exp2(k / 1024.0).astype(np.float32))
+        fn = np.abs(fn)
+    elif kind == "ones":
+        S[:] = 1
+        fn = np.full_like(fn, 2.0 ** -12) * (1 + 2.0 ** -23 * rng.integers(0, 2, fn.shape))
+    elif kind == "cancelling":
+        S[1::2] = -S[::2]
+        fn[:, 1::2] = fn[:, ::2]
+    elif kind == "power_of_two":
+        fn[:, 1:] *= 1e-6
+        S[0] = 1
+        fn[:, 0] = 1
+    elif kind == "tiny":
+        S *= 2.0 ** -60
+        fn *= 2.0 ** -60
+    elif kind == "subnormal":
+        S *= 2.0 ** -70
+        fn *= 2.0 ** -70
+    elif kind == "huge":
+        S *= 2.0 ** 60
+        fn *= 2.0 ** 62
+    elif kind == "steps":
+        S[:] = np.where((k // 512) % 2 == 0, 1.0, -1.0)
+        fn = np.round(fn * 64) / 64
+    elif kind == "zero_crossings":
+        S = bf16_values((np.sin(k / 100.0)).astype(np.float32))
+        fn = np.abs(fn) * 0 + np.float32(0.01)
+        fn += (rng.standard_normal(fn.shape) * 1e-4).astype(np.float32)
+    else:
+        S[rng.random(K) < 0.99] = 0
+    S, fn = S.astype(np.float32), fn.astype(np.float32)
+    sc, base = np.ones(3, np.float32), np.zeros(mix_n, np.float32)
+    b, p, c = (H(v) for v in lib.hc_pre(T(env, S[None]), T(env, fn), T(env, sc), T(env, base),
+                                        mult))
+    ob, op, oc = orc.hc_pre(S, fn, sc, base, mult)
+    assert same_bits(p[0], op) and same_bits(c[0], oc)
+    assert same_bits(b[0], ob)
