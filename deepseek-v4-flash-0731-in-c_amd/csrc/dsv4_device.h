@@ -416,4 +416,34 @@ __device__ __forceinline__ float chain_cols_deep(const float4 *g, const float4 *
   return acc;
 }
 
+// ---------------------------------------------------- split chains ----
+// A chain acc = fmaf(w, x, acc) moves on the grid of acc's binade: as long as
+// every result stays in its binade, a start shifted by d gives every result
+// shifted by d, exactly, if d is a multiple of twice the coarsest grid met
+// (then also ties round alike). So a chain is cut into
+// segments that run at the same time from guesses (the prefix of the products
+// in double, rounded): 8 candidates per segment, the floats base | j around
+// the guess, cover the residues of 8 grid steps, and the true start a then
+// gives the true end r_j + (a - (base | j)) for j = a's low bits, provided
+// |a - (base | j)| is below the smallest distance of the candidate's results
+// from a binade's ends, and no result lies more than two binades above the
+// start (8 grid steps there = 2 of the coarsest). Where that does not hold the
+// segment is run again from its true start, so the result is always the
+// chain's, bit for bit; a start equal to a candidate needs no condition.
+
+// LDS place of a row's column: 16-byte reads of many lanes, each at its own
+// segment's start (a multiple of 16 columns), spread over the banks.
+__host__ __device__ constexpr int sp_at(int c) { return c + 4 * (c >> 6); }
+
+// A start a (bits A) against a record's candidate j of base b with end r and
+// margin m: true, the end and what is left of the margin, if the end follows.
+__device__ __forceinline__ bool sp_step(float a, uint32_t b, float r, float m, float *end,
+                                        float *left) {
+  const uint32_t A = __float_as_uint(a);
+  const float d = a - __uint_as_float(b | (A & 7u));
+  *end = d == 0.0f ? r : r + d;
+  *left = m - fabsf(d) * 1.0001f;
+  return (A >> 23) == (b >> 23) && (d == 0.0f || fabsf(d) < m);
+}
+
 }  // namespace dsv4

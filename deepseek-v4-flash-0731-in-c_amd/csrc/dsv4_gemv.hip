@@ -559,7 +559,7 @@ __global__ __launch_bounds__(64) void k_rowchain(RowChainArgs a) {
 // latency.) The rows of a workgroup share one row block (block a multiple of
 // 16); in a multiple of 32, at most PC_MAXIN.
 #define PC_ROWS 8
-#define PC_MAXIN 4096
+#define PC_MAXIN 2048
 
 // acc + p[0] + ... + p[4 N4 - 1] in order, p in LDS (16-byte aligned): fully
 // unrolled, so every read is one instruction with an immediate offset and
@@ -585,43 +585,6 @@ __device__ __forceinline__ float pc_chain_fixed(const float4 *p4, float acc) {
     acc = acc + c.w;
     asm volatile("" : "+v"(acc)::"memory");
   }
-  return acc;
-}
-
-// The whole row's chain in one unrolled ring (no block boundaries, where the
-// ring would restart), one 384-column load at a time (96 float4, unrolled
-// within the compiler's limit; the loads chained by template recursion):
-// wait(c) returns once the products of columns < c are in LDS, and is called
-// before the first read of each load.
-template <int J0, int N4, typename Wait>
-__device__ __forceinline__ void pc_chain_seg(const float4 *p4, float &acc,
-                                             float4 (&v)[PC_LA + 1], Wait &wait) {
-  constexpr int LA = PC_LA, R = LA + 1;
-#pragma unroll
-  for (int jj = 0; jj < 96; ++jj) {
-    const int j = J0 + jj;
-    if (j >= N4) break;
-    if (j + LA < N4) {
-      if ((j + LA) % 96 == 0) wait(4 * (j + LA) + 4);
-      v[(j + LA) % R] = p4[j + LA];
-    }
-    const float4 c = v[j % R];
-    acc = acc + c.x;
-    acc = acc + c.y;
-    acc = acc + c.z;
-    acc = acc + c.w;
-    asm volatile("" : "+v"(acc)::"memory");
-  }
-  if constexpr (J0 + 96 < N4) pc_chain_seg<J0 + 96, N4>(p4, acc, v, wait);
-}
-
-template <int N4, typename Wait>
-__device__ __forceinline__ float pc_chain_row(const float4 *p4, float acc, Wait &wait) {
-  float4 v[PC_LA + 1];
-  wait(4 * PC_LA);
-#pragma unroll
-  for (int j = 0; j < PC_LA; ++j) v[j] = p4[j];
-  pc_chain_seg<0, N4>(p4, acc, v, wait);
   return acc;
 }
 
@@ -742,21 +705,227 @@ __global__ __launch_bounds__(256) void k_fp8_prodchain(float *__restrict__ y,
     asm volatile("" ::: "memory");  // the product reads stay after the count's
     ready = need;
   };
-  if (n4 == 1024) {  // the model's width: one ring over the whole row
-    acc = pc_chain_row<1024>(p4, acc, wait_cols);
-  } else {
-    int b = 0;
+  int b = 0;
 #pragma unroll 1
-    for (; b + 64 <= n4; b += 64) {
-      wait_cols(4 * (b + 64));
-      acc = pc_chain_fixed<64>(p4 + b, acc);
-    }
-    for (; b + 8 <= n4; b += 8) {
-      wait_cols(4 * (b + 8));
-      acc = pc_chain_fixed<8>(p4 + b, acc);
-    }
+  for (; b + 64 <= n4; b += 64) {
+    wait_cols(4 * (b + 64));
+    acc = pc_chain_fixed<64>(p4 + b, acc);
+  }
+  for (; b + 8 <= n4; b += 8) {
+    wait_cols(4 * (b + 8));
+    acc = pc_chain_fixed<8>(p4 + b, acc);
   }
   y[r0 + tid] = acc;
+}
+
+// The same product chains for longer rows, split (split chains,
+// dsv4_device.h): the products do not depend on the sum, so a row is cut into
+// 64 segments that run at once from guessed starts, and the serial part is a
+// walk over groups of eight segments. A workgroup takes PS_ROWS rows, a wave
+// per row, a lane per segment with all 8 candidates in registers. Thread t
+// forms the products of columns 16 t .. + 15 of every row (its x and scale
+// stay in registers) and their sum in double; lane s then chooses the start of
+// segment s among the middle six multiples of 8 columns of its 64 by the
+// largest |prefix| (by simulation 0.2 segments of a row miss, 3.6 without). The candidates stay within 20 grid steps of the start of each
+// other (7 at the start; a tie may add one step per grid, a coarser grid its
+// own step, at most two binades up), so the margin of the first one less 32
+// steps serves them all. Bound: instruction issue of the candidates' chains
+// (12 per column and segment, on segments as long as the longest of the wave's,
+// about 1.7 times the mean), then the serial walk and the first memory round
+// trip; 2048 x 4096: 15.1 us, 20.9 us as one add chain per row.
+#define PS_ROWS 4
+#define PS_MININ 1024
+#define PS_MAXIN 4096  // 64 segments of 64 columns
+#define PS_REC 10  // dwords per record: r[8], base | binades up, margin
+__host__ __device__ constexpr int ps_pr(int in) { return PS_ROWS * (sp_at(in - 16) + 16); }
+// the products, then the sums of the 16-column chunks (double) and of their
+// first halves (float), whose place the records take
+static size_t ps_lds(int in) { return ((size_t)ps_pr(in) + PS_ROWS * 256 * 3) * 4; }
+
+// acc + the products of columns [c, e), in order (c, e multiples of 8); the
+// next 8 are read while 8 are added.
+__device__ __forceinline__ float ps_chain(const float *p, int c, int e, float acc) {
+  const float4 *q = reinterpret_cast<const float4 *>(p + sp_at(c));
+  float4 v0 = q[0], v1 = q[1];
+  for (; c < e; c += 8) {
+    q = reinterpret_cast<const float4 *>(p + sp_at(min(c + 8, e - 8)));
+    const float4 n0 = q[0], n1 = q[1];
+    acc = acc + v0.x;
+    acc = acc + v0.y;
+    acc = acc + v0.z;
+    acc = acc + v0.w;
+    acc = acc + v1.x;
+    acc = acc + v1.y;
+    acc = acc + v1.z;
+    acc = acc + v1.w;
+    v0 = n0;
+    v1 = n1;
+  }
+  return acc;
+}
+
+template <int MODE>
+__global__ __launch_bounds__(64 * PS_ROWS) void k_fp8_prodsplit(float *__restrict__ y,
+                                                                const float *__restrict__ x,
+                                                                const uint8_t *__restrict__ W,
+                                                                const float *__restrict__ wscale,
+                                                                int in, int rows, int block) {
+  extern __shared__ __align__(16) float lds[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int row = __builtin_amdgcn_readfirstlane(tid >> 6), r0 = blockIdx.x * PS_ROWS;
+  const int cblocks = (in + block - 1) / block, nch = in / 16;
+  const int rs = ps_pr(in) / PS_ROWS;  // product row stride
+  float *rec = lds + ps_pr(in) + row * 64 * PS_REC;
+  double *ps = reinterpret_cast<double *>(lds + ps_pr(in));  // [PS_ROWS][256], before rec
+  float *ph = reinterpret_cast<float *>(ps + PS_ROWS * 256);  // [PS_ROWS][256]
+  if (tid < nch) {
+    float4 xv[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) xv[q] = reinterpret_cast<const float4 *>(x)[4 * tid + q];
+    const float sc = wscale[(size_t)(r0 / block) * cblocks + 16 * tid / block];
+    const BufRsrc rw = buf_rsrc(W + (size_t)r0 * in, (uint32_t)(min(PS_ROWS, rows - r0) * in));
+    uint4 w[PS_ROWS];
+#pragma unroll
+    for (int r = 0; r < PS_ROWS; ++r) w[r] = buf_load16(rw, (uint32_t)(r * in + 16 * tid));
+    if (MODE == 0)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        xv[q] = make_float4(xv[q].x * sc, xv[q].y * sc, xv[q].z * sc, xv[q].w * sc);
+#pragma unroll
+    for (int r = 0; r < PS_ROWS; ++r) {
+      const uint32_t wd[4] = {w[r].x, w[r].y, w[r].z, w[r].w};
+      double sum = 0.0;
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        if (d == 2) ph[r * 256 + tid] = (float)sum;
+        const float2 lo = fp8x2<false>(wd[d]), hi = fp8x2<true>(wd[d]);
+        float4 p = make_float4(lo.x * xv[d].x, lo.y * xv[d].y, hi.x * xv[d].z, hi.y * xv[d].w);
+        if (MODE == 1) p = make_float4(p.x * sc, p.y * sc, p.z * sc, p.w * sc);
+        *reinterpret_cast<float4 *>(lds + r * rs + sp_at(16 * tid) + 4 * d) = p;
+        sum += ((double)p.x + (double)p.y) + ((double)p.z + (double)p.w);
+      }
+      ps[r * 256 + tid] = sum;
+    }
+  }
+  __syncthreads();
+  // ---- lane s: prefixes of its 4 chunks, its segment's start and guess
+  const int nseg = (nch + 3) / 4;
+  int beg = 0;
+  uint32_t base = 0;
+  {
+    double v[4], tot = 0.0;
+    float half[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int at = row * 256 + min(4 * lane + q, nch - 1);
+      v[q] = 4 * lane + q < nch ? ps[at] : 0.0;
+      half[q] = ph[at];
+      tot += v[q];
+    }
+    double inc = tot;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const double u = __shfl_up(inc, o);
+      if (lane >= o) inc += u;
+    }
+    double pre = inc - tot;
+    float best = -1.0f;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const float g = (float)(q % 2 ? pre + (double)half[q / 2] : pre);
+      if (q > 0 && q < 7 && 4 * lane + q / 2 < nch && fabsf(g) > best) {
+        best = fabsf(g);
+        beg = 64 * lane + 8 * q;
+        base = f2u(g) & ~7u;
+      }
+      if (q % 2) pre += v[q / 2];
+    }
+    if (lane == 0 || best < 0.0f) {  // the chain's own start; NaN prefixes
+      beg = 64 * lane;
+      base = 0;
+    }
+  }
+  const int nxt = __shfl_down(beg, 1), end = lane + 1 < nseg ? nxt : in;
+  __syncthreads();  // ps is read; rec takes its place
+  // ---- the segments
+  float mgn = __builtin_inff(), top = 0.0f, r[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) r[j] = u2f(base | j);
+  const float *pr = lds + row * rs;
+  if (lane < nseg) {
+    const float4 *q4 = reinterpret_cast<const float4 *>(pr + sp_at(beg));
+    float4 v[2] = {q4[0], q4[1]};
+    for (int c = beg; c < end; c += 8) {
+      q4 = reinterpret_cast<const float4 *>(pr + sp_at(min(c + 8, end - 8)));
+      const float4 n[2] = {q4[0], q4[1]};
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const float pv[4] = {v[q].x, v[q].y, v[q].z, v[q].w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) r[j] = r[j] + pv[i];
+          // the smaller distance to the binade's ends b, 2 b: b / 2 less that
+          // to its middle (each step exact)
+          const float b = u2f(f2u(r[0]) & 0xFF800000u), mid = fmaf(-1.5f, b, r[0]);
+          mgn = fminf(mgn, fmaf(0.5f, fabsf(b), -fabsf(mid)));
+          top = fmaxf(top, fabsf(r[0]));
+        }
+      }
+      v[0] = n[0];
+      v[1] = n[1];
+    }
+    const int up = (int)(f2u(top) >> 23) - (int)((base >> 23) & 255u);
+    // 32 grid steps of the start: its last place times 32
+    const float step = fabsf(u2f(base | 1u) - u2f(base));
+    const float m = up <= 2 ? mgn * 0.999f - 32.0f * step : 0.0f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) rec[lane * PS_REC + j] = r[j];
+    rec[lane * PS_REC + 8] = u2f(base | (uint32_t)max(0, min(up, 7)));
+    rec[lane * PS_REC + 9] = m > 0.0f ? m : 0.0f;
+  }
+  __syncthreads();
+  // ---- eight segments at a time: lane = (group lane / 8, candidate lane % 8)
+  const int ngrp = (nseg + 7) / 8, s0 = 8 * (lane >> 3);
+  float gend = 0.0f, gm = -1.0f;
+  uint32_t gbase = 0;
+  if (s0 < nseg) {
+    gbase = f2u(rec[s0 * PS_REC + 8]) & ~7u;
+    float a = u2f(gbase | (lane & 7)), m = __builtin_inff();
+    int up = 0;
+    bool ok = true;
+    for (int s = s0; s < min(s0 + 8, nseg); ++s) {
+      const float *R = rec + s * PS_REC;
+      const uint32_t b = f2u(R[8]);
+      float e, left;
+      ok = sp_step(a, b & ~7u, R[f2u(a) & 7], R[9], &e, &left) && ok;
+      up = max(up, (int)(b >> 23 & 255u) + (int)(b & 7u));
+      a = e;
+      m = fminf(m, left);
+    }
+    gend = a;
+    gm = !ok ? -1.0f : up <= (int)(gbase >> 23 & 255u) + 2 && m > 0.0f ? m : 0.0f;
+  }
+  // ---- the walk (every lane the same)
+  float a = 0.0f;
+  for (int q = 0; q < ngrp; ++q) {
+    const int j = __builtin_amdgcn_readfirstlane((int)(f2u(a) & 7u)) + 8 * q;
+    const uint32_t b = (uint32_t)__builtin_amdgcn_readlane((int)gbase, 8 * q);
+    const float m = u2f(__builtin_amdgcn_readlane(f2u(gm), j));
+    float e, left;
+    if (sp_step(a, b, u2f(__builtin_amdgcn_readlane(f2u(gend), j)), m, &e, &left) && m >= 0.0f) {
+      a = e;
+      continue;
+    }
+    for (int s = 8 * q; s < min(8 * q + 8, nseg); ++s) {
+      const float *R = rec + s * PS_REC;
+      if (sp_step(a, f2u(R[8]) & ~7u, R[f2u(a) & 7], R[9], &e, &left))
+        a = e;
+      else
+        a = ps_chain(pr, __builtin_amdgcn_readlane(beg, s), __builtin_amdgcn_readlane(end, s), a);
+    }
+  }
+  if (lane == 0 && r0 + row < rows) y[r0 + row] = a;
 }
 
 // ================================================ batched BF16 rows ====
@@ -1555,6 +1724,19 @@ int dsv4g_gemv_fp8_float(float *y, const float *x, const uint8_t *W, const float
                          int in, int rows, int block, int mode, void *stream) {
   if (in <= 0 || rows <= 0 || block <= 0)
     return dsv4g_fail(DSV4G_EINVAL, "gemv_fp8_float: bad size");
+  // split chains where the row is long, or too ragged for the product chains
+  // (2048 rows of 3008 columns 14 us against 17, of 2048 12.6 against 12.0, of
+  // 1024 11 against 7.5; of 2064 12.5 against 22)
+  if (in % 16 == 0 && (in > PC_MAXIN || (in % 32 && in >= PS_MININ)) && in <= PS_MAXIN &&
+      block % 16 == 0 && ((uintptr_t)x & 15) == 0) {
+    // more than the default 64 KB of LDS (a host-side setting of the kernel)
+    auto k = mode == 0 ? k_fp8_prodsplit<0> : k_fp8_prodsplit<1>;
+    DSV4G_HIP(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)ps_lds(PS_MAXIN)));
+    hipLaunchKernelGGL(k, dim3((unsigned)((rows + PS_ROWS - 1) / PS_ROWS)), dim3(64 * PS_ROWS),
+                       ps_lds(in), (hipStream_t)stream, y, x, W, wscale, in, rows, block);
+    return dsv4g_check_launch("gemv_fp8_float");
+  }
   if (in % 32 == 0 && in <= PC_MAXIN && block % 16 == 0 && ((uintptr_t)x & 15) == 0) {
     const size_t lds = ((size_t)in + (size_t)PC_ROWS * (in + 4) + (in + block - 1) / block) * 4;
     const void *fn = mode == 0 ? (const void *)k_fp8_prodchain<0> : (const void *)k_fp8_prodchain<1>;

@@ -427,19 +427,8 @@ __global__ void __launch_bounds__(64 * NW) k_hc_pre(HcArgs a) {
 }
 
 // ---- few tokens: the chains split.
-// A chain acc = fmaf(w, x, acc) moves on the grid of acc's binade: as long as
-// every result stays in its binade, a start shifted by d gives every result
-// shifted by d, exactly, if d is a multiple of twice the coarsest grid met
-// (then also ties round alike). So the chain of a mix is cut into SEG
-// segments that run at the same time from guesses (the prefix of the products
-// in double, rounded): 8 candidates per segment, the floats base | j around
-// the guess, cover the residues of 8 grid steps, and the true start a then
-// gives the true end r_j + (a - (base | j)) for j = a's low bits, provided
-// |a - (base | j)| is below the smallest distance of the candidate's results
-// from a binade's ends, and no result lies more than two binades above the
-// start (8 grid steps there = 2 of the coarsest). Where that does not hold the
-// segment is run again from its true start, so the result is always the
-// chain's, bit for bit; a start equal to a candidate needs no condition.
+// The 24 mixes are cut into segments that run at once (split chains,
+// dsv4_device.h), a workgroup per mix and token:
 //  - Boundaries: each the multiple of 16 columns with the largest |prefix| of
 //    its 128 columns (a small start has a fine grid, which later results
 //    leave: without the choice 3.6 segments of 128 per chain miss, with it
@@ -462,7 +451,6 @@ constexpr int SP_MINK = 2048;
 constexpr int SP_REC = 13;         // dwords per record: r[8], base, margin[2], top, pad (odd)
 constexpr int SP_SREC = 17;        // per eight segments: end[8], margin[8], pad (odd)
 
-__host__ __device__ constexpr int sp_at(int c) { return c + 4 * (c >> 6); }  // LDS column
 constexpr size_t sp_lds(int K) {
   return ((size_t)2 * sp_at(K) + SP_SEG * SP_REC + SP_SEG / 8 * SP_SREC + 2 * SP_SEG) * 4;
 }
@@ -481,17 +469,6 @@ __device__ __forceinline__ float sp_chain(const float *w, const float *x, int c,
     fma_group(acc, wv, xv);
   }
   return acc;
-}
-
-// A start a (bits A) against a record's candidate j of base b with end r and
-// margin m: true, the end and what is left of the margin, if the end follows.
-__device__ __forceinline__ bool sp_step(float a, uint32_t b, float r, float m, float *end,
-                                        float *left) {
-  const uint32_t A = __float_as_uint(a);
-  const float d = a - __uint_as_float(b | (A & 7u));
-  *end = d == 0.0f ? r : r + d;
-  *left = m - fabsf(d) * 1.0001f;
-  return (A >> 23) == (b >> 23) && (d == 0.0f || fabsf(d) < m);
 }
 
 __global__ void __launch_bounds__(SP_T) k_hc_mix_split(float *__restrict__ bin,

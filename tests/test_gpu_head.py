@@ -244,3 +244,69 @@ def test_bf16_batch_row_tiles(env, rows, batch):
         assert torch.equal(y[t].view(torch.int32), one.view(torch.int32)), t
         last = orc.gemv_bf16(H(x[t]), H(W[-1:]).view(np.uint16), in_, 1, 0)
         assert same_bits(H(y[t, -1:]), last), t
+
+
+@pytest.mark.parametrize("rows,in_,block", [(1, 1024, 128), (5, 1040, 16), (130, 4096, 128),
+                                            (67, 4080, 32), (33, 2064, 48), (16, 1008, 16),
+                                            (12, 4112, 16)])
+def test_fp8_split_rows(env, rows, in_, block):
+    """The split product chains (rows of 1024 to 4096 columns, ragged last
+    segments, groups and workgroups, small blocks) and the widths just outside."""
+    orc, lib = env["orc"], env["lib"]
+    rng = np.random.default_rng(rows + in_)
+    codes = rng.integers(0, 256, (rows, in_)).astype(np.uint8)
+    codes[(codes & 0x7F) == 0x7F] = 0
+    scales = (rng.random(((rows + block - 1) // block, (in_ + block - 1) // block)) + 0.01) \
+        .astype(np.float32)
+    for x in (rng.standard_normal(in_).astype(np.float32),
+              np.ldexp(rng.standard_normal(in_), rng.integers(-30, 30, in_)).astype(np.float32)):
+        for mode, ref in ((0, orc.gemv_fp8_legacy), (1, orc.gemv_fp8_tbl)):
+            y = H(lib.gemv_fp8_float(T(env, x), T(env, codes), T(env, scales), in_, rows, block,
+                                     mode))
+            assert same_bits(y, ref(x, codes, scales, in_, rows, block)), mode
+
+
+@pytest.mark.parametrize("kind", ["zeros", "growing", "ones", "cancelling", "power_of_two",
+                                  "subnormal", "huge", "steps", "ties", "sparse"])
+def test_fp8_split_values(env, kind):
+    """Sums whose segments do not follow from their guesses (as
+    test_hc_pre_split_chain_values): every row bit-exact."""
+    orc, lib = env["orc"], env["lib"]
+    rows, in_ = 12, 4096
+    rng = np.random.default_rng(23)
+    w = (rng.standard_normal((rows, in_)) * 0.02).astype(np.float32)
+    x = rng.standard_normal(in_).astype(np.float32)
+    k = np.arange(in_)
+    if kind == "zeros":
+        x[:] = 0
+    elif kind == "growing":
+        x, w = np.exp2(k / 200.0).astype(np.float32), np.abs(w)
+    elif kind == "ones":
+        x[:], w[:] = 1, 1
+    elif kind == "cancelling":
+        x[1::2], w[:, 1::2] = -x[::2], w[:, ::2]
+    elif kind == "power_of_two":
+        w[:] = 1
+        x = (x * 1e-7).astype(np.float32)
+        x[0] = 1
+    elif kind == "subnormal":
+        x = np.ldexp(x, -140).astype(np.float32)
+    elif kind == "huge":
+        x = np.ldexp(x, 125).astype(np.float32)
+    elif kind == "steps":
+        x[:] = np.where((k // 300) % 2 == 0, 1.0, -1.0)
+        w = np.sign(w) * 0.25 + 0.5
+    elif kind == "ties":  # half a step of the sum's grid at every column
+        w[:] = 1
+        x[:] = 2.0 ** -24
+        x[0] = 1.0
+        x[2000:] *= -1
+    else:
+        x[rng.random(in_) < 0.98] = 0
+    codes, scales = orc.quant_fp8_blocks_absmax(w.astype(np.float32))
+    if kind in ("power_of_two", "ties"):
+        scales[:] = 1.0 / 448.0 * 448.0
+        codes[:] = 0x38  # 1.0
+    for mode, ref in ((0, orc.gemv_fp8_legacy), (1, orc.gemv_fp8_tbl)):
+        y = H(lib.gemv_fp8_float(T(env, x), T(env, codes), T(env, scales), in_, rows, 128, mode))
+        assert same_bits(y, ref(x, codes, scales, in_, rows, 128)), mode
