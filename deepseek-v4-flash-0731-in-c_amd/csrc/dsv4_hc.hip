@@ -4,11 +4,13 @@
 // state in HBM from one layer to the next. Bit-exact with the reference:
 //
 //  - hc_pre (src/dsv4/dsv4_model.c:7123-7156): 24 mixes (mult 4), each an
-//    fmaf chain over mult*hidden = 16384 products in index order. The chains
-//    are run as they are, one lane per chain, in wave 0 of a workgroup per
-//    token; the other waves stream the rows and the state through an LDS ring
-//    in 128-column chunks so the chains never wait on HBM. The kernel's time
-//    is the chain's dependent-FMA latency (16384 steps), not bandwidth.
+//    fmaf chain over mult*hidden = 16384 products in index order. Few tokens:
+//    the chains are cut into segments that run at once (k_hc_mix_split); many:
+//    tiles of chains on the fp32 matrix unit (k_hc_mix_mfma); both leave the
+//    rest to k_hc_finish. Between, and at other shapes, k_hc_pre runs the
+//    chains as they are, one lane per chain, in wave 0 of a workgroup per
+//    token, while the other waves stream the rows and the state through an
+//    LDS ring; its time is the chain's dependent-FMA latency (16384 steps).
 //  - the sums of squares of hc_pre and rmsnorm_bf16 (src/dsv4/dsv4_model.c:
 //    4934-4951) are sequential double sums in the reference. Here they are
 //    summed in parallel; every term is exact (a float squared fits a double),
@@ -623,6 +625,103 @@ __global__ void __launch_bounds__(SP_T) k_hc_mix_split(float *__restrict__ bin,
   if (lane == 0) bin[(size_t)t * hid + mix] = a;
 }
 
+// ---- many tokens: the chains on the fp32 matrix unit.
+// v_mfma_f32_16x16x4 adds its four products one after another, each as one
+// rounded fma, so a tile of 16 mixes x 16 tokens fed four columns at a time
+// runs 256 of the chains bit for bit. A one-wave workgroup takes a tile. Bound:
+// the dependent MFMA's 33 clocks per four columns (16384 columns: 57 us), as
+// long as nothing stands between two of them: a lane loads 16 consecutive
+// columns of a row and of a token MX_D steps of 64 columns ahead, writes them
+// to LDS split by c % 4 (a choice of registers, no instruction) and reads its
+// column c % 4 = lane / 16 of 16 columns back with one 16-byte read, the next
+// step's while this step's 16 MFMAs run. LDS operations of the one wave are in
+// order, so it needs no barrier. Measured 94 us up to 300 tokens, 99 at 777,
+// 117 at 4096 (with k_hc_finish 122 us at 777 tokens; 320 us as one workgroup of
+// chains per token in four rounds).
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+constexpr int MX_D = 4;    // steps of loads in flight
+constexpr int MX_RS = 68;  // LDS floats per row: 64 + 4 (16 rows: distinct banks)
+
+__global__ void __launch_bounds__(64) k_hc_mix_mfma(float *__restrict__ bin,
+                                                    const float *__restrict__ state,
+                                                    const float *__restrict__ fn, int K,
+                                                    int mix_n, int hid, int n) {
+  __shared__ __align__(16) float lw[2][16 * MX_RS], lx[2][16 * MX_RS];
+  const int l = threadIdx.x, l16 = l & 15, g = l >> 4;
+  const int m0 = blockIdx.y * 16, t0 = blockIdx.x * 16;
+  const uint32_t rb = 4u * (uint32_t)K;
+  const BufRsrc rw = buf_rsrc(fn + (size_t)m0 * K, (uint32_t)min(16, mix_n - m0) * rb);
+  const BufRsrc rx = buf_rsrc(state + (size_t)t0 * K, (uint32_t)min(16, n - t0) * rb);
+  // lane = (row l / 4, columns 16 (l % 4) .. + 15 of a step); rows past the
+  // mixes or the tokens are out of range (zeros), steps past K are not used
+  const uint32_t go = (uint32_t)(l >> 2) * rb + 64u * (uint32_t)(l & 3);
+  const int wo = (l >> 2) * MX_RS + 4 * (l & 3), ro = l16 * MX_RS + 16 * g;
+  uint4 W[MX_D][4], X[MX_D][4];
+  auto load = [&](int d, int s) {
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      W[d][q] = buf_load16(rw, go + 256u * (uint32_t)s + 16u * q);
+      X[d][q] = buf_load16(rx, go + 256u * (uint32_t)s + 16u * q);
+    }
+  };
+  auto put = [&](float *dst, const uint4 (&c)[4]) {
+    *(uint4 *)(dst + wo) = make_uint4(c[0].x, c[1].x, c[2].x, c[3].x);
+    *(uint4 *)(dst + wo + 16) = make_uint4(c[0].y, c[1].y, c[2].y, c[3].y);
+    *(uint4 *)(dst + wo + 32) = make_uint4(c[0].z, c[1].z, c[2].z, c[3].z);
+    *(uint4 *)(dst + wo + 48) = make_uint4(c[0].w, c[1].w, c[2].w, c[3].w);
+  };
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f}, a[2][4], b[2][4];
+  auto get = [&](int o, int buf) {
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      a[o][q] = *(const f32x4 *)(lw[buf] + ro + 4 * q);
+      b[o][q] = *(const f32x4 *)(lx[buf] + ro + 4 * q);
+    }
+  };
+#pragma unroll
+  for (int d = 0; d < MX_D; d++) load(d, d);
+  put(lw[0], W[0]);
+  put(lx[0], X[0]);
+  load(0, MX_D);
+  get(0, 0);
+  for (int s0 = 0; s0 < K / 64; s0 += 2 * MX_D) {  // K % (128 MX_D) == 0
+#pragma unroll
+    for (int d = 0; d < 2 * MX_D; d++) {
+      // step s0 + d + 1 into LDS and its operands out of it, its registers
+      // reloaded, beside the MFMAs of step s0 + d
+      const int nd = (d + 1) % MX_D, nb = (d + 1) % 2;
+      put(lw[nb], W[nd]);
+      put(lx[nb], X[nd]);
+      load(nd, s0 + d + 1 + MX_D);
+      get(nb, nb);
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[d % 2][q][e], b[d % 2][q][e], acc, 0, 0, 0);
+      // one MFMA, then what fits into its shadow
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+        __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);  // LDS write
+        __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // load
+        __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);  // VALU
+      }
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // LDS read
+        __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  if (t0 + l16 >= n) return;
+#pragma unroll
+  for (int v = 0; v < 4; v++)
+    if (m0 + 4 * g + v < mix_n) bin[(size_t)(t0 + l16) * hid + m0 + 4 * g + v] = acc[v];
+}
+
 // What follows the mixes (in bin's row): hc_pre's scale, the split, bin and
 // the optional RMSNorm, one workgroup per token.
 constexpr int HF_T = 512;
@@ -730,8 +829,14 @@ bool overlap(const float *a, size_t na, const float *b, size_t nb) {
   return (uintptr_t)a < (uintptr_t)(b + nb) && (uintptr_t)b < (uintptr_t)(a + na);
 }
 
-// Up to this many tokens hc_pre's chains are split over a workgroup per mix.
+// Up to this many tokens hc_pre's chains are split over a workgroup per mix (1
+// token 32 us, 10 37, 32 68, 40 80; a workgroup of chains per token: 83).
 constexpr int HC_SPLIT_TOKENS = 40;
+// From this many tokens on they run on the fp32 matrix unit: up to 256 tokens a
+// workgroup of chains per token takes one round of the CUs (85 us; the matrix
+// unit's 94 us and k_hc_finish), 257 take two (164 us against 112).
+constexpr int HC_MFMA_TOKENS = 257;
+constexpr int MX_MAXK = 1 << 20;  // 16 rows and the run-out within a buffer's 32-bit offsets
 
 }  // namespace
 
@@ -787,17 +892,25 @@ int dsv4g_hc_pre(float *bin, float *post, float *comb, const float *state, const
   a.rms_eps = rms_eps;
   a.hc_eps = hc_eps;
   const int K = mult * hidden, mix_n = (2 + mult) * mult;
-  if (n_tokens <= HC_SPLIT_TOKENS && K % 16 == 0 && K >= SP_MINK && K <= SP_MAXK &&
-      mix_n <= hidden && !overlap(bin, (size_t)n_tokens * hidden, state, (size_t)n_tokens * K) &&
-      !overlap(bin, (size_t)n_tokens * hidden, fn, (size_t)mix_n * K) &&
-      !overlap(bin, (size_t)n_tokens * hidden, scale3, 3) &&
-      !overlap(bin, (size_t)n_tokens * hidden, base, mix_n)) {
-    // more than the default 64 KB of LDS (a host-side setting of the kernel)
-    DSV4G_HIP(hipFuncSetAttribute((const void *)k_hc_mix_split,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  (int)sp_lds(SP_MAXK)));
-    hipLaunchKernelGGL(k_hc_mix_split, dim3(mix_n, n_tokens), dim3(SP_T), sp_lds(K),
-                       (hipStream_t)stream, bin, state, fn, K, mix_n, hidden);
+  const size_t bn = (size_t)n_tokens * hidden;
+  // the mixes pass through bin's rows: bin on its own, and wide enough
+  const bool via_bin = mix_n <= hidden && !overlap(bin, bn, state, (size_t)n_tokens * K) &&
+                       !overlap(bin, bn, fn, (size_t)mix_n * K) && !overlap(bin, bn, scale3, 3) &&
+                       !overlap(bin, bn, base, mix_n);
+  const bool split = n_tokens <= HC_SPLIT_TOKENS && K % 16 == 0 && K >= SP_MINK && K <= SP_MAXK;
+  const bool mfma = n_tokens >= HC_MFMA_TOKENS && K % (128 * MX_D) == 0 && K <= MX_MAXK;
+  if (via_bin && (split || mfma)) {
+    if (split) {
+      // more than the default 64 KB of LDS (a host-side setting of the kernel)
+      DSV4G_HIP(hipFuncSetAttribute((const void *)k_hc_mix_split,
+                                    hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    (int)sp_lds(SP_MAXK)));
+      hipLaunchKernelGGL(k_hc_mix_split, dim3(mix_n, n_tokens), dim3(SP_T), sp_lds(K),
+                         (hipStream_t)stream, bin, state, fn, K, mix_n, hidden);
+    } else {
+      hipLaunchKernelGGL(k_hc_mix_mfma, dim3((n_tokens + 15) / 16, (mix_n + 15) / 16), dim3(64), 0,
+                         (hipStream_t)stream, bin, state, fn, K, mix_n, hidden, n_tokens);
+    }
     hipLaunchKernelGGL(k_hc_finish, dim3(n_tokens), dim3(HF_T), (size_t)hidden * sizeof(float),
                        (hipStream_t)stream, a);
     return dsv4g_check_launch("hc_pre");

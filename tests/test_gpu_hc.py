@@ -255,10 +255,14 @@ def test_ffn_step_full_size(env):
 
 @pytest.mark.parametrize("mult,hid,n", [(4, 4096, 1), (4, 4096, 40), (4, 4096, 41), (1, 2048, 2),
                                         (1, 16384, 1), (2, 1032, 1), (4, 516, 3), (7, 304, 2),
-                                        (3, 5456, 1), (4, 508, 1)])
+                                        (3, 5456, 1), (4, 508, 1), (4, 4096, 256), (4, 4096, 257),
+                                        (4, 128, 300), (2, 256, 259), (7, 512, 273),
+                                        (4, 132, 257)])
 def test_hc_pre_split_chains(env, mult, hid, n):
-    """The chains split over segments (rows of 2048 to 16384 columns, 16 to 63
-    mixes, ragged last segments, up to 40 tokens) and the shapes just outside."""
+    """The chains split over segments (rows of 2048 to 16384 columns, 3 to 63
+    mixes, ragged last segments, up to 40 tokens), on the fp32 matrix unit
+    (from 257 tokens, ragged tiles of mixes and tokens), and the shapes just
+    outside either."""
     orc, lib = env["orc"], env["lib"]
     rng = np.random.default_rng(mult * 1000 + hid + n)
     _, fn, sc, base = hc_inputs(rng, mult, hid)
@@ -266,7 +270,7 @@ def test_hc_pre_split_chains(env, mult, hid, n):
     norm = bf16_bits((1.0 + 0.1 * rng.standard_normal(hid)).astype(np.float32))
     b, p, c = (H(v) for v in lib.hc_pre(T(env, S), T(env, fn), T(env, sc), T(env, base), mult,
                                         T(env, norm)))
-    for t in range(0, n, max(1, n // 8)):
+    for t in sorted({*range(0, n, max(1, n // 8)), n - 1}):
         ob, op, oc = orc.hc_pre(S[t], fn, sc, base, mult)
         assert same_bits(p[t], op) and same_bits(c[t], oc), t
         assert same_bits(b[t], orc.rmsnorm_bf16(ob[None], norm, 1e-6, 1)[0]), t
