@@ -416,6 +416,16 @@ __device__ __forceinline__ float chain_cols_deep(const float4 *g, const float4 *
   return acc;
 }
 
+// LDS tile of 16 rows x 64 columns for the fp32 MFMAs: columns split by
+// c % 4 = g, 16 floats each, whose four 16-byte chunks (columns 16 ch .. + 15)
+// are rotated by row / 4. A wave writing chunk l % 4 of row l / 4 and one
+// reading chunk q of row l % 16 then both touch every bank once per 16 lanes
+// (with rows of 68 floats and no rotation the writes were 4-way conflicts).
+constexpr int MT_RS = 80;  // floats per row
+__device__ __forceinline__ int mt_at(int row, int ch) {
+  return row * MT_RS + 4 * ((ch + (row >> 2)) & 3);
+}
+
 // ---------------------------------------------------- split chains ----
 // A chain acc = fmaf(w, x, acc) moves on the grid of acc's binade: as long as
 // every result stays in its binade, a start shifted by d gives every result

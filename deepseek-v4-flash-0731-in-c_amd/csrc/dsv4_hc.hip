@@ -110,12 +110,36 @@ __device__ __forceinline__ float hc_sigmoid(float x) {
   return e / (1.0f + e);
 }
 
+// Lane 4 a + b of the first 16 lanes holds entry (a, b) of a 4 x 4 matrix: the
+// sums of its row (a quad) or of its column in index order, by DPP (no LDS round
+// trip; with ds_bpermute fetches the split took 6 us). A row rotation by 4 k
+// brings entry (a - k, b), so the lane picks term j as rotation (a - j) % 4.
+template <int CTRL>
+__device__ __forceinline__ float dpp_mov(float v) {
+  return __uint_as_float(
+      __builtin_amdgcn_update_dpp(0, __float_as_uint(v), CTRL, 0xF, 0xF, true));
+}
+__device__ __forceinline__ float sum4_row(float v) {
+  float s = 0.0f;
+  s += dpp_mov<0x00>(v);  // quad_perm: every lane of the quad reads lane j
+  s += dpp_mov<0x55>(v);
+  s += dpp_mov<0xAA>(v);
+  s += dpp_mov<0xFF>(v);
+  return s;
+}
+__device__ __forceinline__ float sum4_col(float v, int a) {
+  const float r1 = dpp_mov<0x124>(v), r2 = dpp_mov<0x128>(v), r3 = dpp_mov<0x12C>(v);  // row_ror
+  const float t0 = a == 0 ? v : a == 1 ? r1 : a == 2 ? r2 : r3;
+  const float t1 = a == 1 ? v : a == 2 ? r1 : a == 3 ? r2 : r3;
+  const float t2 = a == 2 ? v : a == 3 ? r1 : a == 0 ? r2 : r3;
+  const float t3 = a == 3 ? v : a == 0 ? r1 : a == 1 ? r2 : r3;
+  return (((0.0f + t0) + t1) + t2) + t3;
+}
+
 // dsv4_hc_split on the lanes of one wave (call from a whole wave): lane
 // i < m gets pre[i], post[i]; lane a*m + b < m*m gets comb[a][b]. mixes: LDS.
-// M: m when known at compile time (the model's 4), else 0. With M the row and
-// column sums of the Sinkhorn passes fetch their M terms with independent
-// shuffles (one LDS round trip per pass instead of M dependent ones) and add
-// them in index order.
+// M: m when known at compile time (the model's 4, whose Sinkhorn sums go by
+// DPP), else 0.
 template <int M>
 __device__ void hc_split_wave_t(float *pre, float *post, float *comb, const float *mixes,
                                 const float *scale3, const float *base, int m_rt, int iters,
@@ -143,14 +167,10 @@ __device__ void hc_split_wave_t(float *pre, float *post, float *comb, const floa
   // one column pass, then iters-1 (row, column) passes
   for (int pass = 0; pass < 2 * iters - 1; pass++) {
     const bool by_col = (pass & 1) == 0;
-    s = 0.0f;
-    if (M) {
-      float t[M ? M : 1];
-#pragma unroll
-      for (int j = 0; j < M; j++) t[j] = __shfl(v, by_col ? j * M + b : a * M + j);
-#pragma unroll
-      for (int j = 0; j < M; j++) s += t[j];
+    if (M == 4) {
+      s = by_col ? sum4_col(v, a & 3) : sum4_row(v);
     } else {
+      s = 0.0f;
       for (int j = 0; j < m; j++) s += __shfl(v, by_col ? j * m + b : a * m + j);
     }
     v = v / (s + eps);
@@ -635,18 +655,17 @@ __global__ void __launch_bounds__(SP_T) k_hc_mix_split(float *__restrict__ bin,
 // to LDS split by c % 4 (a choice of registers, no instruction) and reads its
 // column c % 4 = lane / 16 of 16 columns back with one 16-byte read, the next
 // step's while this step's 16 MFMAs run. LDS operations of the one wave are in
-// order, so it needs no barrier. Measured 94 us up to 300 tokens, 99 at 777,
-// 117 at 4096 (with k_hc_finish 122 us at 777 tokens; 320 us as one workgroup of
+// order, so it needs no barrier. Measured 82 us up to 300 tokens, 88 at 777,
+// 105 at 4096 (with k_hc_finish 113 us at 777 tokens; 320 us as one workgroup of
 // chains per token in four rounds).
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 constexpr int MX_D = 4;    // steps of loads in flight
-constexpr int MX_RS = 68;  // LDS floats per row: 64 + 4 (16 rows: distinct banks)
 
 __global__ void __launch_bounds__(64) k_hc_mix_mfma(float *__restrict__ bin,
                                                     const float *__restrict__ state,
                                                     const float *__restrict__ fn, int K,
                                                     int mix_n, int hid, int n) {
-  __shared__ __align__(16) float lw[2][16 * MX_RS], lx[2][16 * MX_RS];
+  __shared__ __align__(16) float lw[16 * MT_RS], lx[16 * MT_RS];
   const int l = threadIdx.x, l16 = l & 15, g = l >> 4;
   const int m0 = blockIdx.y * 16, t0 = blockIdx.x * 16;
   const uint32_t rb = 4u * (uint32_t)K;
@@ -655,7 +674,9 @@ __global__ void __launch_bounds__(64) k_hc_mix_mfma(float *__restrict__ bin,
   // lane = (row l / 4, columns 16 (l % 4) .. + 15 of a step); rows past the
   // mixes or the tokens are out of range (zeros), steps past K are not used
   const uint32_t go = (uint32_t)(l >> 2) * rb + 64u * (uint32_t)(l & 3);
-  const int wo = (l >> 2) * MX_RS + 4 * (l & 3), ro = l16 * MX_RS + 16 * g;
+  const int wo = mt_at(l >> 2, l & 3);
+  const int ro[4] = {mt_at(l16, 0) + 16 * g, mt_at(l16, 1) + 16 * g, mt_at(l16, 2) + 16 * g,
+                     mt_at(l16, 3) + 16 * g};
   uint4 W[MX_D][4], X[MX_D][4];
   auto load = [&](int d, int s) {
 #pragma unroll
@@ -671,29 +692,29 @@ __global__ void __launch_bounds__(64) k_hc_mix_mfma(float *__restrict__ bin,
     *(uint4 *)(dst + wo + 48) = make_uint4(c[0].w, c[1].w, c[2].w, c[3].w);
   };
   f32x4 acc = {0.f, 0.f, 0.f, 0.f}, a[2][4], b[2][4];
-  auto get = [&](int o, int buf) {
+  auto get = [&](int o) {
 #pragma unroll
     for (int q = 0; q < 4; q++) {
-      a[o][q] = *(const f32x4 *)(lw[buf] + ro + 4 * q);
-      b[o][q] = *(const f32x4 *)(lx[buf] + ro + 4 * q);
+      a[o][q] = *(const f32x4 *)(lw + ro[q]);
+      b[o][q] = *(const f32x4 *)(lx + ro[q]);
     }
   };
 #pragma unroll
   for (int d = 0; d < MX_D; d++) load(d, d);
-  put(lw[0], W[0]);
-  put(lx[0], X[0]);
+  put(lw, W[0]);
+  put(lx, X[0]);
   load(0, MX_D);
-  get(0, 0);
-  for (int s0 = 0; s0 < K / 64; s0 += 2 * MX_D) {  // K % (128 MX_D) == 0
+  get(0);
+  for (int s0 = 0; s0 < K / 64; s0 += MX_D) {  // K % (64 MX_D) == 0
 #pragma unroll
-    for (int d = 0; d < 2 * MX_D; d++) {
+    for (int d = 0; d < MX_D; d++) {
       // step s0 + d + 1 into LDS and its operands out of it, its registers
       // reloaded, beside the MFMAs of step s0 + d
-      const int nd = (d + 1) % MX_D, nb = (d + 1) % 2;
-      put(lw[nb], W[nd]);
-      put(lx[nb], X[nd]);
+      const int nd = (d + 1) % MX_D;
+      put(lw, W[nd]);
+      put(lx, X[nd]);
       load(nd, s0 + d + 1 + MX_D);
-      get(nb, nb);
+      get((d + 1) % 2);
 #pragma unroll
       for (int q = 0; q < 4; q++)
 #pragma unroll
@@ -723,8 +744,13 @@ __global__ void __launch_bounds__(64) k_hc_mix_mfma(float *__restrict__ bin,
 }
 
 // What follows the mixes (in bin's row): hc_pre's scale, the split, bin and
-// the optional RMSNorm, one workgroup per token.
+// the optional RMSNorm, one workgroup per token. NJ > 0: the thread's 4 NJ
+// columns of all four streams (mult 4, hidden at most 4 NJ HF_T) are kept in
+// registers from the sum of squares on, so the state is read once and the
+// round trip is not paid again behind the split. Bound: launch, that round
+// trip, the split's 39 dependent divisions, two workgroup sums.
 constexpr int HF_T = 512;
+template <int NJ>
 __global__ void __launch_bounds__(HF_T) k_hc_finish(HcArgs a) {
   extern __shared__ __align__(16) float lds[];
   __shared__ float s_mix[64], s_pre[8], s_post[8], s_comb[64], s_scale;
@@ -734,10 +760,29 @@ __global__ void __launch_bounds__(HF_T) k_hc_finish(HcArgs a) {
   const float *state = a.state + (size_t)t * K;
   if (tid < mix_n) s_mix[tid] = a.bin[(size_t)t * hid + tid];
   double ss = 0.0;
-  for (int i = 4 * tid; i < K; i += 4 * HF_T) {
-    const float4 x = *(const float4 *)(state + i);
+  auto square = [&](const float4 &x) {
     const double x0 = x.x, x1 = x.y, x2 = x.z, x3 = x.w;
     ss += x0 * x0 + x1 * x1 + x2 * x2 + x3 * x3;
+  };
+  float4 x[NJ ? NJ : 1][4], gain[NJ ? NJ : 1];
+  if (NJ) {
+#pragma unroll
+    for (int j = 0; j < NJ; j++) {
+      const int c = 4 * (tid + HF_T * j);
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        x[j][i] = c < hid ? *(const float4 *)(state + (size_t)i * hid + c)
+                          : make_float4(0.f, 0.f, 0.f, 0.f);
+      if (a.norm_w && c < hid)
+        gain[j] = make_float4(bf16_to_f32(a.norm_w[c]), bf16_to_f32(a.norm_w[c + 1]),
+                              bf16_to_f32(a.norm_w[c + 2]), bf16_to_f32(a.norm_w[c + 3]));
+    }
+#pragma unroll
+    for (int j = 0; j < NJ; j++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) square(x[j][i]);
+  } else {
+    for (int i = 4 * tid; i < K; i += 4 * HF_T) square(*(const float4 *)(state + i));
   }
   ss = wave_sum_d(ss);
   if (lane == 0) s_part[wave] = ss;
@@ -748,7 +793,53 @@ __global__ void __launch_bounds__(HF_T) k_hc_finish(HcArgs a) {
     hc_scale_split(a, state, t, est, s_mix, s_pre, s_post, s_comb);
   }
   __syncthreads();
-  hc_bin_norm(a, state, t, s_pre, s_part, &s_scale, lds);
+  if (!NJ) {
+    hc_bin_norm(a, state, t, s_pre, s_part, &s_scale, lds);
+    return;
+  }
+  const float p0 = s_pre[0], p1 = s_pre[1], p2 = s_pre[2], p3 = s_pre[3];
+  auto mix = [&](float x0, float x1, float x2, float x3) {
+    return bf16_round(fmaf(p3, x3, fmaf(p2, x2, fmaf(p1, x1, fmaf(p0, x0, 0.0f)))));
+  };
+  float4 bv[NJ ? NJ : 1];
+  ss = 0.0;
+#pragma unroll
+  for (int j = 0; j < NJ; j++) {
+    bv[j] = make_float4(mix(x[j][0].x, x[j][1].x, x[j][2].x, x[j][3].x),
+                        mix(x[j][0].y, x[j][1].y, x[j][2].y, x[j][3].y),
+                        mix(x[j][0].z, x[j][1].z, x[j][2].z, x[j][3].z),
+                        mix(x[j][0].w, x[j][1].w, x[j][2].w, x[j][3].w));
+    if (4 * (tid + HF_T * j) < hid) square(bv[j]);
+  }
+  float r = 1.0f;
+  if (a.norm_w) {
+    ss = wave_sum_d(ss);
+    if (lane == 0) s_part[wave] = ss;
+    __syncthreads();
+    double est = 0.0;
+    for (int w = 0; w < HF_T / 64; w++) est += s_part[w];
+    bool exact;
+    r = rms_scale_bounded(est, hid, a.rms_eps, &exact);
+    if (!exact) {  // the same in every thread: the sum in index order
+#pragma unroll
+      for (int j = 0; j < NJ; j++)
+        if (4 * (tid + HF_T * j) < hid) *(float4 *)(lds + 4 * (tid + HF_T * j)) = bv[j];
+      __syncthreads();
+      double s2 = 0.0;
+      for (int c = 0; c < hid; c++) s2 += (double)lds[c] * (double)lds[c];
+      r = rms_scale(s2, hid, a.rms_eps);
+    }
+  }
+  float *out = a.bin + (size_t)t * hid;
+#pragma unroll
+  for (int j = 0; j < NJ; j++) {
+    const int c = 4 * (tid + HF_T * j);
+    if (c >= hid) continue;
+    const float o[4] = {bv[j].x, bv[j].y, bv[j].z, bv[j].w};
+    const float gn[4] = {gain[j].x, gain[j].y, gain[j].z, gain[j].w};
+#pragma unroll
+    for (int i = 0; i < 4; i++) out[c + i] = a.norm_w ? bf16_round(o[i] * r * gn[i]) : o[i];
+  }
 }
 
 // rmsnorm_bf16 over rows of x (one workgroup per row); y may alias x.
@@ -834,7 +925,7 @@ bool overlap(const float *a, size_t na, const float *b, size_t nb) {
 constexpr int HC_SPLIT_TOKENS = 40;
 // From this many tokens on they run on the fp32 matrix unit: up to 256 tokens a
 // workgroup of chains per token takes one round of the CUs (85 us; the matrix
-// unit's 94 us and k_hc_finish), 257 take two (164 us against 112).
+// unit's 82 us and k_hc_finish), 257 take two (164 us against 100).
 constexpr int HC_MFMA_TOKENS = 257;
 constexpr int MX_MAXK = 1 << 20;  // 16 rows and the run-out within a buffer's 32-bit offsets
 
@@ -898,7 +989,7 @@ int dsv4g_hc_pre(float *bin, float *post, float *comb, const float *state, const
                        !overlap(bin, bn, fn, (size_t)mix_n * K) && !overlap(bin, bn, scale3, 3) &&
                        !overlap(bin, bn, base, mix_n);
   const bool split = n_tokens <= HC_SPLIT_TOKENS && K % 16 == 0 && K >= SP_MINK && K <= SP_MAXK;
-  const bool mfma = n_tokens >= HC_MFMA_TOKENS && K % (128 * MX_D) == 0 && K <= MX_MAXK;
+  const bool mfma = n_tokens >= HC_MFMA_TOKENS && K % (64 * MX_D) == 0 && K <= MX_MAXK;
   if (via_bin && (split || mfma)) {
     if (split) {
       // more than the default 64 KB of LDS (a host-side setting of the kernel)
@@ -911,7 +1002,11 @@ int dsv4g_hc_pre(float *bin, float *post, float *comb, const float *state, const
       hipLaunchKernelGGL(k_hc_mix_mfma, dim3((n_tokens + 15) / 16, (mix_n + 15) / 16), dim3(64), 0,
                          (hipStream_t)stream, bin, state, fn, K, mix_n, hidden, n_tokens);
     }
-    hipLaunchKernelGGL(k_hc_finish, dim3(n_tokens), dim3(HF_T), (size_t)hidden * sizeof(float),
+    // (777 tokens, three rounds of workgroups: 25 us without the registers, 31
+    // with; 1 token 12.6 and 11.4, 300 tokens 16.6 and 15.6)
+    hipLaunchKernelGGL(mult == 4 && hidden <= 8 * HF_T && n_tokens <= 512 ? k_hc_finish<2>
+                                                                          : k_hc_finish<0>,
+                       dim3(n_tokens), dim3(HF_T), (size_t)hidden * sizeof(float),
                        (hipStream_t)stream, a);
     return dsv4g_check_launch("hc_pre");
   }
