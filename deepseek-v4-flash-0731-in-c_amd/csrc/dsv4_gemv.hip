@@ -14,6 +14,8 @@ using namespace dsv4;
 
 namespace dsv4 {
 
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
 // ============================================================ activation ==
 // One wave per 128-element group (src/dsv4/dsv4_model.c:5580-5606).
 // grid = (ceil(n/128), nvec); x/qx rows are n apart, qscale rows ceil(n/128).
@@ -335,6 +337,176 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(G == 4 ? 4 
     }
     __syncthreads();  // LDS is refilled by the next group
   }
+}
+
+// Several tokens on the fp32 matrix unit: an MFMA 16x16x4 adds its four
+// products in column order, each as one rounded fma (k_bf16_rows_mfma), so a
+// tile started from zero at every 128-column block runs the block's chains of
+// 16 rows x 16 tokens bit for bit. Every block's partials go to LDS, and a
+// thread per (row, token) chains the (partial, scale) pairs in order, so the
+// blocks are independent: KS waves share a row tile (wave k: blocks k, k + KS,
+// ...) where the rows alone leave SIMDs idle (4096 rows: 256 tiles), 4 / KS
+// tiles per workgroup. Each wave stages for itself, without barriers (its LDS
+// operations are in order): a lane loads 16 consecutive columns of a row and
+// of a token, FM_D steps of 64 columns ahead, writes them to LDS widened and
+// split by c % 4 (a choice of registers) and reads its column of 16 back with
+// one 16-byte read, the next step's while this step's MFMAs run. Bound: the
+// MFMA's latency where a SIMD has one wave, then the matrix rate, on tokens
+// padded to 16. in a multiple of 128. Token groups of one row tile are
+// neighbours on one XCD: its weights come from that L2 after the first.
+#define FM_D 4
+template <int KS>
+static size_t fp8_mfma_lds(int CB) {
+  return ((size_t)4 * 2 * 16 * MT_RS + (size_t)(4 / KS) * CB * 257 + (size_t)CB * 16) * 4;
+}
+
+template <int KS>
+__global__ __launch_bounds__(256) void k_fp8_proj_mfma(GemvArgs a, int nvec, int units,
+                                                       int groups) {
+  constexpr int NT = 4 / KS;  // row tiles per workgroup
+  extern __shared__ __align__(16) float lds[];
+  const int tid = threadIdx.x, l = tid & 63, l16 = l & 15, g = l >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), tl = wave / KS, ks = wave % KS;
+  const int mat = blockIdx.z, in = a.in, CB = in / 128;
+  const int k8 = blockIdx.x >> 3;
+  const int unit = (k8 / groups) * 8 + (blockIdx.x & 7), t0 = (k8 % groups) * 16;
+  if (unit >= units) return;
+  const int r0 = unit * 16 * NT, nt = min(16, nvec - t0);
+  float *lw = lds + wave * 2 * 16 * MT_RS, *lx = lw + 16 * MT_RS;
+  float *parts = lds + 4 * 2 * 16 * MT_RS;                    // [NT][CB][256]
+  float *sq = parts + (size_t)NT * CB * 256;                  // [CB][16]
+  uint32_t *sw = reinterpret_cast<uint32_t *>(sq + CB * 16);  // [NT][CB]
+  const int wr0 = r0 + 16 * tl;  // this wave's rows
+  const int nrow = __builtin_amdgcn_readfirstlane(max(0, min(16, a.rows - wr0)));
+  const BufRsrc rw = buf_rsrc(a.W[mat] + (size_t)wr0 * in, (uint32_t)nrow * (uint32_t)in);
+  const BufRsrc rx = buf_rsrc(a.qx + (size_t)t0 * a.qx_stride,
+                              4u * ((uint32_t)(nt - 1) * (uint32_t)a.qx_stride + (uint32_t)in));
+  // lane = (row l / 4, columns 16 (l % 4) .. + 15 of a step); rows past the
+  // matrix or the tokens are out of range (zeros), blocks past the width not
+  // stored
+  const uint32_t wo = (uint32_t)(l >> 2) * (uint32_t)in + 16u * (uint32_t)(l & 3);
+  const uint32_t xo = (l >> 2) < nt ? 4u * (uint32_t)(l >> 2) * (uint32_t)a.qx_stride +
+                                          64u * (uint32_t)(l & 3)
+                                    : 0x80000000u;
+  const int po = mt_at(l >> 2, l & 3);
+  const int ro[4] = {mt_at(l16, 0) + 16 * g, mt_at(l16, 1) + 16 * g, mt_at(l16, 2) + 16 * g,
+                     mt_at(l16, 3) + 16 * g};
+  uint4 W[FM_D], X[FM_D][4];
+  auto load = [&](int d, int i) {  // step i: half i % 2 of block ks + KS (i / 2)
+    const uint32_t c = 128u * (uint32_t)(ks + KS * (i >> 1)) + 64u * (uint32_t)(i & 1);
+    W[d] = buf_load16(rw, wo + c);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) X[d][q] = buf_load16(rx, xo + 4u * c + 16u * q);
+  };
+  auto put = [&](int d) {
+    const uint32_t wd[4] = {W[d].x, W[d].y, W[d].z, W[d].w};
+    float2 lo[4], hi[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      lo[q] = fp8x2<false>(wd[q]);
+      hi[q] = fp8x2<true>(wd[q]);
+    }
+    *reinterpret_cast<float4 *>(lw + po) = make_float4(lo[0].x, lo[1].x, lo[2].x, lo[3].x);
+    *reinterpret_cast<float4 *>(lw + po + 16) = make_float4(lo[0].y, lo[1].y, lo[2].y, lo[3].y);
+    *reinterpret_cast<float4 *>(lw + po + 32) = make_float4(hi[0].x, hi[1].x, hi[2].x, hi[3].x);
+    *reinterpret_cast<float4 *>(lw + po + 48) = make_float4(hi[0].y, hi[1].y, hi[2].y, hi[3].y);
+    const uint4 *c = X[d];
+    *reinterpret_cast<uint4 *>(lx + po) = make_uint4(c[0].x, c[1].x, c[2].x, c[3].x);
+    *reinterpret_cast<uint4 *>(lx + po + 16) = make_uint4(c[0].y, c[1].y, c[2].y, c[3].y);
+    *reinterpret_cast<uint4 *>(lx + po + 32) = make_uint4(c[0].z, c[1].z, c[2].z, c[3].z);
+    *reinterpret_cast<uint4 *>(lx + po + 48) = make_uint4(c[0].w, c[1].w, c[2].w, c[3].w);
+  };
+  f32x4 av[2][4], bv[2][4];
+  auto get = [&](int o) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      av[o][q] = *reinterpret_cast<const f32x4 *>(lw + ro[q]);
+      bv[o][q] = *reinterpret_cast<const f32x4 *>(lx + ro[q]);
+    }
+  };
+#pragma unroll
+  for (int d = 0; d < FM_D; ++d) load(d, d);
+  for (int i = tid; i < CB * 16; i += 256) {
+    const int t = i & 15;
+    sq[i] = t < nt ? a.qscale[(size_t)(t0 + t) * a.qs_stride + (i >> 4)] : 0.0f;
+  }
+  for (int i = tid; i < NT * CB; i += 256) {
+    const int r = min(r0 + 16 * (i / CB), a.rows - 1);
+    sw[i] = a.S[mat][(size_t)(r / 128) * CB + i % CB];
+  }
+  put(0);
+  load(0, FM_D);
+  get(0);
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int i0 = 0; ks + KS * (i0 >> 1) < CB; i0 += FM_D) {
+#pragma unroll
+    for (int d = 0; d < FM_D; ++d) {
+      // the next step into LDS and its operands out of it, its registers
+      // reloaded, beside the MFMAs of step i0 + d
+      const int nd = (d + 1) % FM_D;
+      put(nd);
+      load(nd, i0 + d + 1 + FM_D);
+      get((d + 1) % 2);
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av[d % 2][q][e], bv[d % 2][q][e], acc, 0, 0,
+                                                     0);
+      // one MFMA, then what fits into its shadow
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+        __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);  // LDS write
+        __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // load
+        __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);  // VALU
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // LDS read
+        __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (d % 2) {  // the block's end
+        const int cb = ks + KS * ((i0 + d) >> 1);
+        if (cb < CB)  // uniform
+          *reinterpret_cast<f32x4 *>(parts + ((size_t)tl * CB + cb) * 256 + 16 * l16 + 4 * g) =
+              acc;
+        acc = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+    }
+  }
+  __syncthreads();
+  // thread i: row i % 16 of the tile, token i / 16
+  const int tok = tid >> 4;
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int row = r0 + 16 * t + (tid & 15);
+    if (row >= a.rows || tok >= nt) continue;
+    float o = 0.0f;
+#pragma unroll 8
+    for (int cb = 0; cb < CB; ++cb) {
+      const uint32_t sc = sw[t * CB + cb];
+      const float n =
+          fmaf(parts[((size_t)t * CB + cb) * 256 + tid], sq[cb * 16 + tok] * e8m0(sc), o);
+      o = sc == 255u ? o : n;  // NaN scale: the reference skips the block
+    }
+    a.y[mat][(size_t)(t0 + tok) * a.y_stride + row] = a.round_out ? bf16_round(o) : o;
+  }
+}
+
+template <int KS>
+static int launch_fp8_proj_mfma(const GemvArgs *a, int nvec, int nmat, hipStream_t st) {
+  const int CB = a->in / 128, rt = 16 * (4 / KS);
+  const int units = (a->rows + rt - 1) / rt, groups = (nvec + 15) / 16;
+  const size_t lds = fp8_mfma_lds<KS>(CB);
+  if (lds > 64 * 1024)  // (a host-side setting of the kernel)
+    DSV4G_HIP(hipFuncSetAttribute((const void *)k_fp8_proj_mfma<KS>,
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)(140 * 1024)));
+  hipLaunchKernelGGL(k_fp8_proj_mfma<KS>, dim3((units + 7) / 8 * 8 * groups, 1, nmat), dim3(256),
+                     lds, st, *a, nvec, units, groups);
+  return 0;
 }
 
 // Token groups per workgroup: all of them when the row tiles alone give
@@ -955,8 +1127,10 @@ __global__ __launch_bounds__(64 * PS_ROWS) void k_fp8_prodsplit(float *__restric
 //
 // ROUTER: the gate's rows; y is the scores sqrt(softplus(z)), choice the
 // scores plus the bias, and blockIdx.y the token tile.
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-#define RM_XS 68  // LDS floats per token of an x tile: 64 + 4 (16 tokens: distinct banks)
+// LDS floats per token of an x tile: 64 + 4. (Rows of 80 floats with rotated
+// chunks, mt_at, write without conflicts, but leave fewer workgroups per CU: 80000
+// rows, 64 tokens 347 -> 427 us.)
+#define RM_XS 68
 template <int NT, int MR, bool ROUTER>
 __global__ __launch_bounds__(256, 2) void k_bf16_rows_mfma(float *__restrict__ y,
                                                            const float *__restrict__ x,
@@ -1547,6 +1721,25 @@ int dsv4g_launch_gemv_fp8(const GemvArgs *a, int nvec, int nmat, void *stream) {
   // (and the four tokens' activations fit LDS beside the rest: in <= 2048)
   const bool many = nvec > 1 && a->in <= 2048 &&
                     (long)(a->rows + 256 / sl - 1) / (256 / sl) * nmat >= 1024;
+  // Several tokens on the matrix unit where it is the faster by these fits (us).
+  // Matrix unit: a round of workgroups costs 1.4 per block of a wave with a CU
+  // each (in > 1024: 4 waves share a row tile: 8192 columns x 4096 rows 24, 46,
+  // 66 for 16, 32, 33 tokens; 4096 x 1024 13), 2.3 with two workgroups on a CU
+  // (1024 x 32768: 20, 41, 56). VALU: 0.083 per token and million weights, 0.052
+  // four tokens at a time (8192 x 4096 rows: 5 tokens 21.7, 8 30.7, 16 52, 33 97;
+  // 1024 x 32768: 8 tokens 19.6, 16 32, 33 63; 4096 x 1024: 16 tokens 11, 33 17).
+  if (nvec > 1 && a->in % 128 == 0) {
+    const int ks = CB > 8 ? 4 : 1;
+    const long wgs = (a->rows + 64 / ks - 1L) / (64 / ks) * ((nvec + 15) / 16) * nmat;
+    const double mfma = ks == 4 ? 2 + 1.4 * ((CB + 3) / 4) * ((wgs + 255) / 256)
+                                : 2 + 2.3 * CB * ((wgs + 511) / 512);
+    const double valu = 5 + (many ? 0.052 : 0.083) * 1e-6 * nvec * nmat * a->rows * a->in;
+    if (mfma < valu) {
+      DSV4G_TRY(ks == 4 ? launch_fp8_proj_mfma<4>(a, nvec, nmat, st)
+                        : launch_fp8_proj_mfma<1>(a, nvec, nmat, st));
+      return dsv4g_check_launch("gemv_fp8");
+    }
+  }
   switch (sl * (many ? 10 : 1)) {
     case 8: launch_fp8_proj<8, 1>(a, nvec, nmat, st); break;
     case 16: launch_fp8_proj<16, 1>(a, nvec, nmat, st); break;

@@ -94,3 +94,25 @@ def test_pair(env):
                                  T(env, S1), cols, rows)
     w0, w1 = orc.gemv_fp8_pair_q(qx, qs, W0, S0, W1, S1, cols, rows)
     assert same_bits(y0.cpu().numpy(), w0) and same_bits(y1.cpu().numpy(), w1)
+
+
+@pytest.mark.parametrize("rows,cols,n", [(1, 128, 2), (70, 128, 17), (333, 384, 16), (130, 1024, 40),
+                                         (1000, 1024, 33), (2100, 1152, 33), (2050, 2048, 33),
+                                         (1040, 8192, 21), (1024, 4096, 23), (1024, 4096, 24)])
+def test_several_tokens(env, rows, cols, n):
+    """Both sides of the rule between the VALU's and the matrix unit's chains:
+    one to 64 blocks a row, ragged row tiles, workgroups and token groups, a
+    NaN scale, with and without rounding; every token of sampled rows."""
+    orc, lib = env["orc"], env["lib"]
+    rng = np.random.default_rng(rows + cols + n)
+    W, S = fp8_weights(orc, rng, rows, cols, nan_block=True)
+    x = rng.standard_normal((n, cols)).astype(np.float32)
+    qx, qs = orc.quant_fp8_act(x)
+    chk = np.unique(np.r_[0, rows - 1, rng.integers(0, rows, 40)])
+    for ro in (1, 0):
+        y = lib.gemv_fp8_batch_q(T(env, qx), T(env, qs), T(env, W), T(env, S), cols, rows,
+                                 round_out=ro).cpu().numpy()
+        for t in range(n):
+            want = np.array([orc.gemv_fp8_q(qx[t], qs[t], W[k:k + 1], S[k // 128:k // 128 + 1],
+                                            cols, 1, ro)[0] for k in chk], np.float32)
+            assert same_bits(y[t][chk], want), (t, ro)
