@@ -896,6 +896,36 @@ __global__ void __launch_bounds__(256) k_hc_post(float *state, const float *bran
   }
 }
 
+// The same for mult 4 with four columns per thread (16-byte loads and stores;
+// hid a multiple of 4, state and branch 16-byte aligned). Bound: HBM, the state
+// read and written once (777 tokens, 113 MB).
+__global__ void __launch_bounds__(64) k_hc_post4(float *state, const float *branch,
+                                                 const float *post, const float *comb, int hid) {
+  const int t = blockIdx.y, c = 4 * (blockIdx.x * 64 + threadIdx.x);
+  if (c >= hid) return;
+  float *st = state + (size_t)t * 4 * hid + c;
+  const float *po = post + (size_t)t * 4, *cb = comb + (size_t)t * 16;
+  float4 old[4];
+#pragma unroll
+  for (int k = 0; k < 4; k++) old[k] = *(const float4 *)(st + (size_t)k * hid);
+  const float4 br = *(const float4 *)(branch + (size_t)t * hid + c);
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const float p = po[i];
+    float4 y = make_float4(p * br.x, p * br.y, p * br.z, p * br.w);
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const float m = cb[4 * i + k];
+      y.x = fmaf(m, old[k].x, y.x);
+      y.y = fmaf(m, old[k].y, y.y);
+      y.z = fmaf(m, old[k].z, y.z);
+      y.w = fmaf(m, old[k].w, y.w);
+    }
+    *(float4 *)(st + (size_t)i * hid) =
+        make_float4(bf16_round(y.x), bf16_round(y.y), bf16_round(y.z), bf16_round(y.w));
+  }
+}
+
 // dsv4_hc_split for n independent rows of mixes (one wave each).
 __global__ void __launch_bounds__(64) k_hc_split(float *pre, float *post, float *comb,
                                                  const float *mixes, const float *scale3,
@@ -1032,6 +1062,11 @@ int dsv4g_hc_post(float *state, const float *branch, const float *post, const fl
       n_tokens < 0)
     return dsv4g_fail(DSV4G_EINVAL, "hc_post: bad arguments (mult 1..%d)", HC_MAX_MULT);
   if (n_tokens == 0) return 0;
+  if (mult == 4 && hidden % 4 == 0 && aligned16(state) && aligned16(branch)) {
+    hipLaunchKernelGGL(k_hc_post4, dim3((hidden + 255) / 256, n_tokens), dim3(64), 0,
+                       (hipStream_t)stream, state, branch, post, comb, hidden);
+    return dsv4g_check_launch("hc_post");
+  }
   hipLaunchKernelGGL(k_hc_post, dim3((hidden + 255) / 256, n_tokens), dim3(256), 0,
                      (hipStream_t)stream, state, branch, post, comb, mult, hidden);
   return dsv4g_check_launch("hc_post");

@@ -330,3 +330,23 @@ def test_hc_pre_split_chain_values(env, kind):
     ob, op, oc = orc.hc_pre(S, fn, sc, base, mult)
     assert same_bits(p[0], op) and same_bits(c[0], oc)
     assert same_bits(b[0], ob)
+
+
+@pytest.mark.parametrize("hid,off", [(4, 0), (260, 0), (4100, 0), (256, 1), (255, 0)])
+def test_hc_post_four_columns(env, hid, off):
+    """mult 4: four columns per thread (ragged last workgroups), and the one-column
+    form for a state off 16-byte alignment or an odd width."""
+    orc, lib, torch = env["orc"], env["lib"], env["torch"]
+    rng = np.random.default_rng(hid)
+    n = 3
+    S = bf16_values(rng.standard_normal((n, 4 * hid)).astype(np.float32))
+    br = bf16_values(rng.standard_normal((n, hid)).astype(np.float32))
+    post = (rng.random((n, 4)) * 2).astype(np.float32)
+    comb = rng.random((n, 16)).astype(np.float32)
+    st = torch.zeros(n * 4 * hid + off, dtype=torch.float32, device=env["dev"])[off:]
+    st = st.view(n, 4 * hid)
+    st.copy_(T(env, S))
+    lib.hc_post(st, T(env, br), T(env, post), T(env, comb), 4)
+    got = H(st)
+    for t in range(n):
+        assert same_bits(got[t], orc.hc_post(S[t], br[t], post[t], comb[t], 4)), t
