@@ -44,10 +44,9 @@ sys.path.insert(0, os.path.join(ROOT, "deepseek-v4-flash-0731-in-c_amd", "python
 HBM_PEAK_GBS = 8000.0
 BF16_PEAK_TFLOPS = 2500.0   # dense MFMA peaks of one MI355X
 FP8_PEAK_TFLOPS = 5000.0
-# fp32 vector FMA: 256 CUs x 64 lanes x 2 flops x 2.4 GHz issued one FMA per
-# lane per clock; the published 157.3 TFLOP/s is the packed (two-wide) rate,
-# which this build does not emit
-FP32_FMA_PEAK_TFLOPS = 78.6
+# fp32 matrix unit (V_MFMA_F32_16X16X4, whose chains are exact fmaf chains):
+# 256 CUs x 4 SIMDs x 1024 FMA per 32 clocks x 2 flops x 2.4 GHz.
+FP32_MFMA_PEAK_TFLOPS = 157.3
 VOCAB = 129280
 METRIC = "MoE layer decode GB/s (% HBM peak); prefill grouped-GEMM TFLOPS (% MFMA)"
 
@@ -218,11 +217,11 @@ def bench_fp8_matvec(lib, cpu_seconds):
          "roofline": {"bound": "chain latency", "achieved": round(gbs, 1),
                       "peak": HBM_PEAK_GBS, "unit": "GB/s",
                       "frac": round(gbs / HBM_PEAK_GBS, 4)},
-         "note": "the products w*xs of 8 rows per workgroup are formed into LDS by all "
-                 "waves; one lane per row then runs the reference's 4096 dependent adds "
-                 "in column order (about 3.7 ns per add when fed from LDS, 2.6 from "
-                 "registers), starting once the first half's products are in LDS: the "
-                 "chain, not the 8.4 MB, bounds the call"}
+         "note": "the products w*xs of 4 rows per workgroup are formed into LDS; the "
+                 "reference's 4096 dependent adds of a row run as 64 segments at once from "
+                 "guessed starts (exact: translation on the sum's grid, segments that do "
+                 "not follow run again): issue of those chains and the serial walk bound "
+                 "the call"}
     if cpu_seconds and cpu_available():
         ref = cpu_ref()
         xh, ch, sh = x.cpu().numpy(), codes[0].cpu().numpy(), scales[0].cpu().numpy()
@@ -349,9 +348,9 @@ def bench_ffn_step(lib, layers, cpu_seconds):
                       "achieved": round(pre_bytes / (ms_pre * 1e-3) / 1e9, 1),
                       "peak": HBM_PEAK_GBS, "unit": "GB/s",
                       "frac": round(pre_bytes / (ms_pre * 1e-3) / 1e9 / HBM_PEAK_GBS, 5),
-                      "note": "hc_pre streams 1.6 MB but its 16384-step dependent chains bound "
-                              "it: 2.05-2.4 ns per step for a lone chain from registers on "
-                              "gfx950 (a floor of about 34 us)"}}
+                      "note": "hc_pre streams 1.6 MB; its 16384-step chains run as 128 segments "
+                              "at once from guessed starts (exact), a workgroup per mix, then "
+                              "one workgroup for the split, bin and the RMSNorm"}}
     if cpu_seconds and cpu_available():
         threads, _ = host_cores()
         set_omp_threads(threads)
@@ -487,8 +486,8 @@ def bench_vocab_head(lib, cpu_seconds):
     wbytes = VOCAB * H * 2
     res = {"workload": "vocabulary head 129280 x 4096 BF16, fp32 logits (dsv4_gemv_bf16; "
                        "1 token: coalesced 64 x 64 tiles transposed through LDS, a lane per "
-                       "row, HBM-bound; 64 tokens: 4 rows x 16 tokens of chains per lane, x "
-                       "from LDS, fp32-FMA-bound)", "weight_bytes": wbytes}
+                       "row, HBM-bound; 64 tokens: the chains as 16 x 16 tiles of the fp32 "
+                       "matrix unit, fp32-MFMA-bound)", "weight_bytes": wbytes}
     for n in (1, 64):
         ms = graph_time(lambda i, n=n: lib.gemv_bf16_into(Y[:n], X[:n], Wu, H, VOCAB, 0),
                         8 if n == 1 else 2)
@@ -501,10 +500,10 @@ def bench_vocab_head(lib, cpu_seconds):
             r["roofline"] = {"bound": "hbm", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS,
                              "unit": "GB/s", "frac": round(gbs / HBM_PEAK_GBS, 4)}
         else:
-            r["roofline"] = {"bound": "fp32 fma issue (the per-row chains are fmaf in column "
-                                      "order, so no matrix-core form is exact)",
-                             "achieved": round(tf, 2), "peak": FP32_FMA_PEAK_TFLOPS,
-                             "unit": "TFLOP/s", "frac": round(tf / FP32_FMA_PEAK_TFLOPS, 4),
+            r["roofline"] = {"bound": "fp32 matrix rate (V_MFMA_F32_16X16X4 adds its products "
+                                      "one after another, so the per-row chains are exact)",
+                             "achieved": round(tf, 2), "peak": FP32_MFMA_PEAK_TFLOPS,
+                             "unit": "TFLOP/s", "frac": round(tf / FP32_MFMA_PEAK_TFLOPS, 4),
                              "hbm_frac": round(gbs / HBM_PEAK_GBS, 4)}
         res[f"{n}_token" + ("s" if n > 1 else "")] = r
     if cpu_seconds and cpu_available():
