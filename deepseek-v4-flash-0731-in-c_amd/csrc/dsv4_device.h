@@ -436,9 +436,9 @@ __device__ __forceinline__ int mt_at(int row, int ch) {
 // the guess, cover the residues of 8 grid steps, and the true start a then
 // gives the true end r_j + (a - (base | j)) for j = a's low bits, provided
 // |a - (base | j)| is below the smallest distance of the candidate's results
-// from a binade's ends, and no result lies more than two binades above the
-// start (8 grid steps there = 2 of the coarsest). Where that does not hold the
-// segment is run again from its true start, so the result is always the
+// from a binade's ends, and no result is infinite or more than two binades
+// above the start (8 grid steps there = 2 of the coarsest). Where that does not
+// hold the segment is run again from its true start, so the result is always the
 // chain's, bit for bit; a start equal to a candidate needs no condition.
 
 // LDS place of a row's column: 16-byte reads of many lanes, each at its own

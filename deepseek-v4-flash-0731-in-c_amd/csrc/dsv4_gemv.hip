@@ -1047,7 +1047,10 @@ __global__ __launch_bounds__(64 * PS_ROWS) void k_fp8_prodsplit(float *__restric
       v[0] = n[0];
       v[1] = n[1];
     }
-    const int up = (int)(f2u(top) >> 23) - (int)((base >> 23) & 255u);
+    // binades up; an infinite result (its distances are NaN, which the minimum
+    // drops) allows no shift
+    const int te = (int)(f2u(top) >> 23);
+    const int up = te < 255 ? te - (int)((base >> 23) & 255u) : 7;
     // 32 grid steps of the start: its last place times 32
     const float step = fabsf(u2f(base | 1u) - u2f(base));
     const float m = up <= 2 ? mgn * 0.999f - 32.0f * step : 0.0f;

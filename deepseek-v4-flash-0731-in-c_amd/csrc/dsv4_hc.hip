@@ -590,8 +590,10 @@ __global__ void __launch_bounds__(SP_T) k_hc_mix_split(float *__restrict__ bin,
         }
       }
     }
-    // no result more than two binades above the start, else no shift at all
-    const bool grid = (__float_as_uint(top) >> 23) <= ((base >> 23) & 255u) + 2u;
+    // no result infinite or more than two binades above the start, else no
+    // shift at all (an infinite one leaves NaN distances, which the minimum drops)
+    const uint32_t te = __float_as_uint(top) >> 23;
+    const bool grid = te < 255u && te <= ((base >> 23) & 255u) + 2u;
     const float m = mgn * 0.999f - spread * 1.001f;
     float *R = rec + s * SP_REC;
 #pragma unroll

@@ -277,12 +277,16 @@ def test_hc_pre_split_chains(env, mult, hid, n):
 
 
 @pytest.mark.parametrize("kind", ["zeros", "growing", "ones", "cancelling", "power_of_two",
-                                  "tiny", "subnormal", "huge", "steps", "zero_crossings", "sparse"])
+                                  "tiny", "subnormal", "huge", "steps", "zero_crossings", "sparse",
+                                  "overflow"])
 def test_hc_pre_split_chain_values(env, kind):
     """Sums whose segments do not follow from their guesses: exact zeros, sums
     that double from segment to segment, ties at every step, sums that return
-    to zero, that stay at a power of two, subnormal and overflowing sums. The
-    mixes reach the outputs through post and comb (scale 1, base 0)."""
+    to zero, that stay at a power of two, subnormal and overflowing sums, and
+    sums just inside the fp32 range whose guesses overflow (terms that the chain
+    loses, then one that takes only the guess past it; both signs). The
+    mixes reach the outputs through post and comb (scale 1, base 0; where they
+    are near 2^128, scale 2^-126)."""
     orc, lib = env["orc"], env["lib"]
     mult, hid = 4, 4096
     K, mix_n = mult * hid, 24
@@ -321,10 +325,17 @@ def test_hc_pre_split_chain_values(env, kind):
         S = bf16_values((np.sin(k / 100.0)).astype(np.float32))
         fn = np.abs(fn) * 0 + np.float32(0.01)
         fn += (rng.standard_normal(fn.shape) * 1e-4).astype(np.float32)
+    elif kind == "overflow":
+        S[:], fn[:] = 1, 0
+        fn[:, 0], fn[:, 1:600] = 1.5 * 2.0 ** 126, 0.4 * 2.0 ** 103
+        fn[:, K - 20] = 2.0 ** 127 + 2.0 ** 125 - 2.0 ** 110
+        fn[::2] *= -1
     else:
         S[rng.random(K) < 0.99] = 0
     S, fn = S.astype(np.float32), fn.astype(np.float32)
     sc, base = np.ones(3, np.float32), np.zeros(mix_n, np.float32)
+    if kind == "overflow":
+        sc[:] = 2.0 ** -126
     b, p, c = (H(v) for v in lib.hc_pre(T(env, S[None]), T(env, fn), T(env, sc), T(env, base),
                                         mult))
     ob, op, oc = orc.hc_pre(S, fn, sc, base, mult)

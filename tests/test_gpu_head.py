@@ -267,10 +267,14 @@ def test_fp8_split_rows(env, rows, in_, block):
 
 
 @pytest.mark.parametrize("kind", ["zeros", "growing", "ones", "cancelling", "power_of_two",
-                                  "subnormal", "huge", "steps", "ties", "sparse"])
+                                  "subnormal", "huge", "steps", "ties", "sparse",
+                                  "overflow"])
 def test_fp8_split_values(env, kind):
     """Sums whose segments do not follow from their guesses (as
-    test_hc_pre_split_chain_values): every row bit-exact."""
+    test_hc_pre_split_chain_values): every row bit-exact. "overflow": the first
+    product, then terms below half a step that the chain loses and a guess
+    counts, then one that takes the guess past the fp32 range and the chain
+    just below it, in both signs."""
     orc, lib = env["orc"], env["lib"]
     rows, in_ = 12, 4096
     rng = np.random.default_rng(23)
@@ -301,12 +305,19 @@ def test_fp8_split_values(env, kind):
         x[:] = 2.0 ** -24
         x[0] = 1.0
         x[2000:] *= -1
+    elif kind == "overflow":
+        x[:] = 0
+        x[0], x[1:600] = 1.5 * 2.0 ** 126, 0.4 * 2.0 ** 103
+        x[in_ - 20] = 2.0 ** 127 + 2.0 ** 125 - 2.0 ** 110
     else:
         x[rng.random(in_) < 0.98] = 0
     codes, scales = orc.quant_fp8_blocks_absmax(w.astype(np.float32))
-    if kind in ("power_of_two", "ties"):
+    if kind in ("power_of_two", "ties", "overflow"):
         scales[:] = 1.0 / 448.0 * 448.0
         codes[:] = 0x38  # 1.0
+    if kind == "overflow":
+        codes[rows // 2:] = 0xB8  # -1.0
+        assert np.isfinite(orc.gemv_fp8_legacy(x, codes, scales, in_, rows, 128)).all()
     for mode, ref in ((0, orc.gemv_fp8_legacy), (1, orc.gemv_fp8_tbl)):
         y = H(lib.gemv_fp8_float(T(env, x), T(env, codes), T(env, scales), in_, rows, 128, mode))
         assert same_bits(y, ref(x, codes, scales, in_, rows, 128)), mode
