@@ -998,6 +998,9 @@ int dsv4g_hc_pre(float *bin, float *post, float *comb, const float *state, const
   if (!aligned16(state) || !aligned16(fn))
     return dsv4g_fail(DSV4G_EINVAL, "hc_pre: state and fn must be 16-byte aligned");
   if (n_tokens == 0) return 0;
+  // every route holds a token's bin row in LDS (k_hc_finish, k_hc_pre)
+  if ((size_t)hidden * sizeof(float) > HC_LDS_BUDGET)
+    return dsv4g_fail(DSV4G_EINVAL, "hc_pre: hidden %d too large", hidden);
   HcArgs a;
   a.bin = bin;
   a.post = post;
@@ -1043,9 +1046,7 @@ int dsv4g_hc_pre(float *bin, float *post, float *comb, const float *state, const
     return dsv4g_check_launch("hc_pre");
   }
   const size_t ring = (size_t)a.ring * ((2 + mult) * mult + 1) * HC_RS * sizeof(float);
-  const size_t lds = std::max(ring, (size_t)hidden * sizeof(float));
-  if (lds > HC_LDS_BUDGET)
-    return dsv4g_fail(DSV4G_EINVAL, "hc_pre: hidden %d too large", hidden);
+  const size_t lds = std::max(ring, (size_t)hidden * sizeof(float));  // ring: hc_ring
   // mult <= 4: 8 waves, 6 of them producers (19 float4 each); larger mult:
   // 4 waves, 2 producers (48 float4 each)
   const int rows = (2 + mult) * mult + 1;

@@ -193,3 +193,18 @@ def test_tiny_checkpoint_hc_weights(orc, ref):
         b = ref.hc_pre(state, fn, sc, base, 2)
         assert all(same_bits(u, v) for u, v in zip(a, b))
         assert same_bits(orc.rmsnorm_bf16(a[0][None], norm), ref.rmsnorm_bf16(b[0][None], norm))
+
+
+@pytest.mark.parametrize("mult,hidden,n", [(4, 38404, 1), (4, 38404, 41), (4, 38464, 257),
+                                           (4, 40960, 257), (4, 262144, 300), (1, 38656, 257)])
+def test_hc_pre_refuses_wide_hidden(mult, hidden, n):
+    """A token's bin row is held in LDS: above 38400 columns hc_pre is refused
+    before anything is launched, whatever route the token count takes. The
+    addresses are never used."""
+    import ctypes as C
+
+    from dsv4_gpu import GpuLib
+    lib = GpuLib().lib
+    a = [C.c_void_p(k << 44) for k in range(1, 8)]
+    rc = lib.dsv4g_hc_pre(*a, None, mult, hidden, 20, 1e-6, 1e-6, n, None, None)
+    assert rc == 1 and b"too large" in lib.dsv4g_last_error()
