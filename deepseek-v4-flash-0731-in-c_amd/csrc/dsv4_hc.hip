@@ -469,7 +469,6 @@ __global__ void __launch_bounds__(64 * NW) k_hc_pre(HcArgs a) {
 constexpr int SP_T = 1024;         // threads, and 16-column pieces at most
 constexpr int SP_SEG = 128;        // segments: 8 pieces each (fewer for a shorter row)
 constexpr int SP_MAXK = 16 * SP_T;
-constexpr int SP_MINK = 2048;
 constexpr int SP_REC = 13;         // dwords per record: r[8], base, margin[2], top, pad (odd)
 constexpr int SP_SREC = 17;        // per eight segments: end[8], margin[8], pad (odd)
 
@@ -955,6 +954,20 @@ bool overlap(const float *a, size_t na, const float *b, size_t nb) {
 // Up to this many tokens hc_pre's chains are split over a workgroup per mix (1
 // token 32 us, 10 37, 32 68, 40 80; a workgroup of chains per token: 83).
 constexpr int HC_SPLIT_TOKENS = 40;
+
+// Whether the split is the faster, by these fits (us) of what the two do not
+// share: a round of workgroups (two on a CU while their LDS allows it, rows to
+// 8606 columns) takes 10 and 0.35 per 1000 columns, the chains 4.1 per 1000.
+// Rows of 2048 columns: 22 (split) against 19 at one token, 34.5 against 20 at
+// 40; of 4096, 24 mixes: 25 against 28.7 at 21 tokens, 33 against 28.7 at 22; of
+// 14336, 63 mixes: 77 against 98 at 12 tokens, 172 against 97.5 at 40; of 16384,
+// 24 mixes: 74 against 80 at 40.
+bool split_pays(int K, int mix_n, int n) {
+  const long wgs = (long)mix_n * n, at_once = sp_lds(K) <= 80 * 1024 ? 512 : 256;
+  const long rounds = (wgs + at_once - 1) / at_once;
+  return (double)rounds * (10 + 0.35e-3 * K) + 2 < 4.1e-3 * K;
+}
+
 // From this many tokens on they run on the fp32 matrix unit: up to 256 tokens a
 // workgroup of chains per token takes one round of the CUs (85 us; the matrix
 // unit's 82 us and k_hc_finish), 257 take two (164 us against 100).
@@ -1023,7 +1036,8 @@ int dsv4g_hc_pre(float *bin, float *post, float *comb, const float *state, const
   const bool via_bin = mix_n <= hidden && !overlap(bin, bn, state, (size_t)n_tokens * K) &&
                        !overlap(bin, bn, fn, (size_t)mix_n * K) && !overlap(bin, bn, scale3, 3) &&
                        !overlap(bin, bn, base, mix_n);
-  const bool split = n_tokens <= HC_SPLIT_TOKENS && K % 16 == 0 && K >= SP_MINK && K <= SP_MAXK;
+  const bool split = n_tokens <= HC_SPLIT_TOKENS && K % 16 == 0 && K <= SP_MAXK &&
+                     split_pays(K, mix_n, n_tokens);
   const bool mfma = n_tokens >= HC_MFMA_TOKENS && K % (64 * MX_D) == 0 && K <= MX_MAXK;
   if (via_bin && (split || mfma)) {
     if (split) {

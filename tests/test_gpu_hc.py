@@ -257,12 +257,14 @@ def test_ffn_step_full_size(env):
                                         (1, 16384, 1), (2, 1032, 1), (4, 516, 3), (7, 304, 2),
                                         (3, 5456, 1), (4, 508, 1), (4, 4096, 256), (4, 4096, 257),
                                         (4, 128, 300), (2, 256, 259), (7, 512, 273),
-                                        (4, 132, 257)])
+                                        (4, 132, 257), (4, 816, 1), (1, 3280, 40),
+                                        (2, 2056, 5), (4, 1024, 21), (4, 1024, 22), (7, 512, 8),
+                                        (7, 512, 9), (7, 2048, 12), (7, 2048, 18)])
 def test_hc_pre_split_chains(env, mult, hid, n):
-    """The chains split over segments (rows of 2048 to 16384 columns, 3 to 63
-    mixes, ragged last segments, up to 40 tokens), on the fp32 matrix unit
-    (from 257 tokens, ragged tiles of mixes and tokens), and the shapes just
-    outside either."""
+    """The chains split over segments (rows of 3264 to 16384 columns, 3 to 63
+    mixes, ragged last segments, up to 40 tokens, both sides of the rounds of
+    workgroups where that pays), on the fp32 matrix unit (from 257 tokens, ragged
+    tiles of mixes and tokens), and the shapes just outside either."""
     orc, lib = env["orc"], env["lib"]
     rng = np.random.default_rng(mult * 1000 + hid + n)
     _, fn, sc, base = hc_inputs(rng, mult, hid)
