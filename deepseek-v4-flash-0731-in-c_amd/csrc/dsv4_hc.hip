@@ -110,36 +110,13 @@ __device__ __forceinline__ float hc_sigmoid(float x) {
   return e / (1.0f + e);
 }
 
-// Lane 4 a + b of the first 16 lanes holds entry (a, b) of a 4 x 4 matrix: the
-// sums of its row (a quad) or of its column in index order, by DPP (no LDS round
-// trip; with ds_bpermute fetches the split took 6 us). A row rotation by 4 k
-// brings entry (a - k, b), so the lane picks term j as rotation (a - j) % 4.
-template <int CTRL>
-__device__ __forceinline__ float dpp_mov(float v) {
-  return __uint_as_float(
-      __builtin_amdgcn_update_dpp(0, __float_as_uint(v), CTRL, 0xF, 0xF, true));
-}
-__device__ __forceinline__ float sum4_row(float v) {
-  float s = 0.0f;
-  s += dpp_mov<0x00>(v);  // quad_perm: every lane of the quad reads lane j
-  s += dpp_mov<0x55>(v);
-  s += dpp_mov<0xAA>(v);
-  s += dpp_mov<0xFF>(v);
-  return s;
-}
-__device__ __forceinline__ float sum4_col(float v, int a) {
-  const float r1 = dpp_mov<0x124>(v), r2 = dpp_mov<0x128>(v), r3 = dpp_mov<0x12C>(v);  // row_ror
-  const float t0 = a == 0 ? v : a == 1 ? r1 : a == 2 ? r2 : r3;
-  const float t1 = a == 1 ? v : a == 2 ? r1 : a == 3 ? r2 : r3;
-  const float t2 = a == 2 ? v : a == 3 ? r1 : a == 0 ? r2 : r3;
-  const float t3 = a == 3 ? v : a == 0 ? r1 : a == 1 ? r2 : r3;
-  return (((0.0f + t0) + t1) + t2) + t3;
-}
-
 // dsv4_hc_split on the lanes of one wave (call from a whole wave): lane
 // i < m gets pre[i], post[i]; lane a*m + b < m*m gets comb[a][b]. mixes: LDS.
-// M: m when known at compile time (the model's 4, whose Sinkhorn sums go by
-// DPP), else 0.
+// M: m when known at compile time (the model's 4), else 0. With M the row and
+// column sums of the Sinkhorn passes fetch their M terms with independent
+// shuffles (one LDS round trip per pass instead of M dependent ones) and add
+// them in index order. (By DPP, whose column sums pick each term out of three
+// rotations, the split took 0.65 us more: 39 dependent passes of selects.)
 template <int M>
 __device__ void hc_split_wave_t(float *pre, float *post, float *comb, const float *mixes,
                                 const float *scale3, const float *base, int m_rt, int iters,
@@ -167,10 +144,14 @@ __device__ void hc_split_wave_t(float *pre, float *post, float *comb, const floa
   // one column pass, then iters-1 (row, column) passes
   for (int pass = 0; pass < 2 * iters - 1; pass++) {
     const bool by_col = (pass & 1) == 0;
-    if (M == 4) {
-      s = by_col ? sum4_col(v, a & 3) : sum4_row(v);
+    s = 0.0f;
+    if (M) {
+      float t[M ? M : 1];
+#pragma unroll
+      for (int j = 0; j < M; j++) t[j] = __shfl(v, by_col ? j * M + b : a * M + j);
+#pragma unroll
+      for (int j = 0; j < M; j++) s += t[j];
     } else {
-      s = 0.0f;
       for (int j = 0; j < m; j++) s += __shfl(v, by_col ? j * m + b : a * m + j);
     }
     v = v / (s + eps);
@@ -1051,8 +1032,8 @@ int dsv4g_hc_pre(float *bin, float *post, float *comb, const float *state, const
       hipLaunchKernelGGL(k_hc_mix_mfma, dim3((n_tokens + 15) / 16, (mix_n + 15) / 16), dim3(64), 0,
                          (hipStream_t)stream, bin, state, fn, K, mix_n, hidden, n_tokens);
     }
-    // (777 tokens, three rounds of workgroups: 25 us without the registers, 31
-    // with; 1 token 12.6 and 11.4, 300 tokens 16.6 and 15.6)
+    // (777 tokens, three rounds of workgroups: 24.4 us without the registers,
+    // about 30 with; 1 token 12.4 and 10.5, 300 tokens 16.5 and 15.0)
     hipLaunchKernelGGL(mult == 4 && hidden <= 8 * HF_T && n_tokens <= 512 ? k_hc_finish<2>
                                                                           : k_hc_finish<0>,
                        dim3(n_tokens), dim3(HF_T), (size_t)hidden * sizeof(float),
