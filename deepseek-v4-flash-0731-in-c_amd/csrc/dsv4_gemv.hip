@@ -1361,9 +1361,10 @@ __global__ __launch_bounds__(64) void k_bf16_rows_tiled(float *__restrict__ y,
 // v with logits[v] > logits[best] in order; so the first index of the
 // largest value, NaNs never taken, and 0 when logits[0] is NaN. One
 // workgroup per row. Bound: one CU's load rate and latency (517 KB per row
-// at the model's vocabulary), so 16 waves with AM_Q 16-byte loads each in
+// at the model's vocabulary), so 16 waves with 8 16-byte loads each in
 // flight: 147 us with 4 waves and one 4-byte load in flight each, about 8 us
-// now (one row of 129280). A thread's loads past the row are clamped to
+// now (one row of 129280); fewer waves and loads for shorter rows
+// (dsv4g_argmax). A thread's loads past the row are clamped to
 // the row's last 4 values (seen twice, which changes nothing). Each thread
 // keeps the first largest value of its ascending indices (bi < 0: none above
 // -inf; a row with no value above -inf gives 0, as the rule does whether
@@ -1376,8 +1377,8 @@ __device__ __forceinline__ void am_merge(float &bv, int &bi, float ov, int oi) {
   }
 }
 
-#define AM_T 1024  // threads per row
-#define AM_Q 8     // 16-byte loads in flight per thread
+// T threads per row, Q 16-byte loads in flight per thread.
+template <int AM_T, int AM_Q>
 __global__ __launch_bounds__(AM_T) void k_argmax(int *idx, const float *logits, int vocab,
                                                  size_t stride) {
   __shared__ float s_v[AM_T / 64];
@@ -1911,8 +1912,15 @@ int dsv4g_argmax(int *idx, const float *logits, int vocab, int n, size_t stride,
                  void *stream) {
   if (!idx || !logits || vocab <= 0 || n <= 0 || stride < (size_t)vocab)
     return dsv4g_fail(DSV4G_EINVAL, "argmax: bad arguments");
-  hipLaunchKernelGGL(k_argmax, dim3((unsigned)n), dim3(AM_T), 0, (hipStream_t)stream, idx,
-                     logits, vocab, stride);
+  // The threads that a row fills: clamped loads cost their issue, and idle waves
+  // their start (8192 rows of 1000: 66 us with 16 waves of 8 loads, 9 with 4 of 1;
+  // of 64: 66 and 4.4). Rows to 16384 take 4 waves up to four times round: 8192
+  // rows of 16384 88 us against 95, one 3.4 against 4.8.
+  const int kind = vocab <= 256 ? 0 : vocab <= 1024 ? 1 : vocab <= 16384 ? 2 : 3;
+  auto k = kind == 0 ? k_argmax<64, 1> : kind == 1 ? k_argmax<256, 1>
+         : kind == 2 ? k_argmax<256, 4> : k_argmax<1024, 8>;
+  hipLaunchKernelGGL(k, dim3((unsigned)n), dim3(kind == 0 ? 64 : kind == 3 ? 1024 : 256), 0,
+                     (hipStream_t)stream, idx, logits, vocab, stride);
   return dsv4g_check_launch("argmax");
 }
 

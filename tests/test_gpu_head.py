@@ -176,10 +176,11 @@ def test_expert_forward_shapes(env, hidden, inter):
     assert same_bits(H(out), ref)
 
 
-@pytest.mark.parametrize("vocab", [1, 2, 3, 4, 5, 7, 4095, 4097, 32767, 32768, 32769, 32771,
-                                   129280])
+@pytest.mark.parametrize("vocab", [1, 2, 3, 4, 5, 7, 255, 256, 257, 1023, 1024, 1025, 4095, 4097,
+                                   16383, 16384, 16385, 32767, 32768, 32769, 32771, 129280])
 def test_greedy_row_lengths(env, vocab):
-    """Rows around the 4-value loads and the 32768-value rounds, rows that start
+    """Rows around the 4-value loads, the sizes where more waves or loads begin
+    (256, 1024, 16384) and the rounds of 4096 and 32768 values, rows that start
     at any float (stride = an odd vocab), the maximum at the first, the last
     and a clamped position, ties across the clamp, and rows of -inf and NaN."""
     lib, torch = env["lib"], env["torch"]
