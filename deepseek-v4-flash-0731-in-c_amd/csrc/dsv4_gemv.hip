@@ -1281,8 +1281,8 @@ __global__ __launch_bounds__(256, 2) void k_bf16_rows_mfma(float *__restrict__ y
   }
 }
 
-// The same chains for 1 or 2 tokens of a large matrix, where HBM is the bound: a
-// lane per output row reading its own row would touch 64 cache lines per load,
+// The same chains for a few tokens of many or narrow rows (tiled_width), where HBM
+// or the launch is the bound: a lane per output row reading its own row would touch 64 cache lines per load,
 // so the wave loads tiles of 64 rows x 64 columns coalesced (lane l: rows
 // 8 i + l / 8, 16 bytes at column 8 (l % 8)), writes them to LDS (rows 144
 // bytes apart, so that the lanes' row reads hit distinct banks) and reads back
@@ -1628,6 +1628,33 @@ static void launch_rows_mfma(float *y, const float *x, const uint16_t *W, int in
     launch_rows_mfma_nt<4>(y, x, W, in, out, round_out, t0, n, st);
 }
 
+// The widest rows that n tokens take through the tiled chains. Those wait on
+// memory and their own latency, about the same time however many waves a CU has,
+// and issue an fma per token and column; the matrix unit's wait less and cost as
+// much for one token as for 16, once per workgroup of 64 rows, so many rows (w =
+// 64-row tiles per CU) favour the tiled form and wide rows or more tokens the
+// matrix unit's (us, tiled / matrix unit). One token: 16384 rows of 128 3.5 / 4.0,
+// of 256 5.3 / 4.7; 40000 of 384 10.0 / 11.5, of 512 15.7 / 13.6; 72000 of 512
+// 20.1 / 21.4, of 4096 163 / 147; 88000 of 4096 171 / 173; 114688 of 4096 176 /
+// 205. Two: 24000 of 192 5.4 / 6.2, of 256 6.7 / 6.6; 96000 of 512 23.8 / 25.2,
+// of 1024 45.2 / 44.2; 100000 of 1024 45.6 / 50.7, of 4096 198 / 195. Three:
+// 50000 of 256 8.9 / 10.3; 100000 of 768 38.8 / 39.6, of 1024 53 / 51. Four:
+// 65536 of 192 7.5 / 10, of 256 12.0 / 11.0. Eight: 65536 of 64 4.7 / 7.1, of 128
+// 9.0 / 8.6; 100000 of 128 10.0 / 13.1, of 192 15.9 / 15.9. (16 tokens of 64
+// columns: 8.8 by tiles of four rows a lane, 12.7 here, at 100000 rows; a shape
+// without a use.)
+static int tiled_width(int n, int out) {
+  constexpr int ANY = 0x7fffffff;
+  //                             w = 1    2    3    4    5    6     7   more
+  static constexpr int W[5][8] = {{128, 384, 384, 384, 512, ANY, ANY, ANY},   // 1 token
+                                  {64, 192, 320, 320, 384, 512, 1024, ANY},   // 2
+                                  {64, 128, 192, 256, 256, 384, 768, 768},    // 3
+                                  {64, 64, 192, 192, 192, 192, 384, 384},     // 4
+                                  {0, 64, 64, 64, 128, 128, 128, 128}};       // 8
+  if (n > 4 && n != 8) return 0;
+  return W[n == 8 ? 4 : n - 1][std::min((out + 16383L) / 16384, 8L) - 1];
+}
+
 // Every (token, expert) score and choice of the batched router, [T][E], exact.
 // Token tiles per wave: the fewest with at most one workgroup per CU (256
 // experts: 38 us up to 400 tokens, 47 at 777, 77 at 2048, 119 at 4096 beside
@@ -1859,21 +1886,21 @@ int dsv4g_gemv_bf16(float *y, const float *x, const uint16_t *W, int in, int out
   if (in <= 0 || out <= 0 || batch <= 0) return dsv4g_fail(DSV4G_EINVAL, "gemv_bf16: bad size");
   const size_t xb = (size_t)batch * in * 4;
   if (in % 64 == 0 && ((uintptr_t)x & 15) == 0 && (size_t)64 * in * 2 < 0xFFFF0000u) {
-    // runs of up to 64 tokens through the matrix unit's chains; 1 or 2 tokens
-    // of a large matrix through the tiled chains (129280 rows: 1 token 185 us
-    // against 227, 2 tokens 223 against 230 to 250, but 3 tokens 245 against
-    // 240; one token of 110000 rows 186 against 176, of 65536 rows 143 against
-    // 107, of 16384 rows 95 against 39), and so do rows too wide for a run's x
-    // within one buffer range, two tokens at a time
+    // runs of up to 64 tokens through the matrix unit's chains, or the tiled
+    // chains where those are the faster (tiled_width); rows too wide for a run's x
+    // within one buffer range go through the tiled chains two tokens at a time
     const bool wide = (size_t)64 * in * 4 >= 0xFFFF0000u;
     for (int t0 = 0; t0 < batch;) {
       const int n = std::min(batch - t0, wide ? 2 : 64);
-      if (wide || (n <= 2 && out > 114688))
-        hipLaunchKernelGGL(n == 1 ? k_bf16_rows_tiled<1> : k_bf16_rows_tiled<2>,
-                           dim3((out + 63) / 64), dim3(64), 0, (hipStream_t)stream, y, x, W, in,
+      if (wide || in <= tiled_width(n, out)) {
+        auto k = n == 1 ? k_bf16_rows_tiled<1> : n == 2 ? k_bf16_rows_tiled<2>
+               : n == 3 ? k_bf16_rows_tiled<3> : n == 4 ? k_bf16_rows_tiled<4>
+                        : k_bf16_rows_tiled<8>;
+        hipLaunchKernelGGL(k, dim3((out + 63) / 64), dim3(64), 0, (hipStream_t)stream, y, x, W, in,
                            out, round_out, t0);
-      else
+      } else {
         launch_rows_mfma(y, x, W, in, out, round_out, t0, n, (hipStream_t)stream);
+      }
       DSV4G_TRY(dsv4g_check_launch("gemv_bf16"));
       t0 += n;
     }

@@ -227,15 +227,14 @@ def test_f32_mfma_is_fma_chain(env, kind):
 @pytest.mark.parametrize("rows,batch", [(16384, 64), (32768 + 5, 4), (65537, 49), (129280, 17),
                                         (129280, 48), (16384, 33), (130, 128), (1, 16),
                                         (114688, 2), (114689, 2), (114689, 65), (114689, 66)])
-def test_bf16_batch_row_tiles(env, rows, batch):
+def test_bf16_batch_row_tiles(env, rows, batch, in_=192):
     """1, 2 and 4 row tiles per wave by the number of rows, 1 to 4 token tiles,
     ragged in both, runs of 64, an odd number of 64-column steps: every token
     equal to its one-token result, and the last row's to the host's chain.
-    Above 114688 rows 1 or 2 tokens take the tiled chains."""
+    A few tokens of many rows take the tiled chains."""
     orc, lib, torch, dev = env["orc"], env["lib"], env["torch"], env["dev"]
     g = torch.Generator(device=dev)
     g.manual_seed(rows + batch)
-    in_ = 192
     W = (torch.randn(rows, in_, generator=g, device=dev) * 0.05).to(torch.bfloat16) \
         .view(torch.int16).contiguous()
     x = torch.randn(batch, in_, generator=g, device=dev)
@@ -245,6 +244,18 @@ def test_bf16_batch_row_tiles(env, rows, batch):
         assert torch.equal(y[t].view(torch.int32), one.view(torch.int32)), t
         last = orc.gemv_bf16(H(x[t]), H(W[-1:]).view(np.uint16), in_, 1, 0)
         assert same_bits(H(y[t, -1:]), last), t
+
+
+@pytest.mark.parametrize("rows,in_,batch", [(17, 64, 4), (16384, 128, 1), (16384, 192, 1),
+                                            (16385, 64, 8), (16385, 128, 3), (16385, 192, 3),
+                                            (40000, 192, 4), (40000, 256, 68), (40000, 320, 2), (40000, 384, 2),
+                                            (70000, 512, 1), (82000, 128, 8), (82000, 128, 7),
+                                            (82000, 576, 65), (98305, 768, 3), (98305, 1024, 2)])
+def test_bf16_narrow_rows(env, rows, in_, batch):
+    """Both sides of the rule between the tiled chains (1, 2, 3, 4 or 8 tokens,
+    whole batches and what a run of 64 leaves) and the matrix unit's, by the
+    number of rows and their width."""
+    test_bf16_batch_row_tiles(env, rows, batch, in_)
 
 
 @pytest.mark.parametrize("rows,in_,block", [(1, 1024, 128), (5, 1040, 16), (130, 4096, 128),
