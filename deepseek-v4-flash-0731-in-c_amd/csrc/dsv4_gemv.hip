@@ -1125,7 +1125,7 @@ __global__ __launch_bounds__(64 * PS_ROWS) void k_fp8_prodsplit(float *__restric
 // 63 -> 47 us); more row tiles as they are (144 bytes apart: conflict-free),
 // read back per (row, 8 columns), v_perm widening the lane's column of each
 // four, which the other tiles' MFMAs cover. x is staged once per workgroup,
-// split by c % 4 as well, double-buffered where 64 KB of LDS allow. The x
+// split by c % 4 as well, double-buffered. The x
 // loads of a step are issued ahead of its weights (loads complete in order).
 //
 // ROUTER: the gate's rows; y is the scores sqrt(softplus(z)), choice the
@@ -1145,9 +1145,8 @@ __global__ __launch_bounds__(256, 2) void k_bf16_rows_mfma(float *__restrict__ y
     t0 = blockIdx.y * 16 * NT;
     nt = min(16 * NT, nt - t0);
   }
-  constexpr int XB = NT * MR == 16 ? 1 : 2;  // x buffers (64 KB of LDS in all)
-  constexpr int D = NT * MR <= 2 ? 4 : 2;    // steps in flight
-  __shared__ __align__(16) float xs[XB][16 * NT * RM_XS];
+  constexpr int D = NT * MR <= 2 ? 4 : 2;  // steps in flight
+  __shared__ __align__(16) float xs[2][16 * NT * RM_XS];
   constexpr bool WIDE = MR == 1;
   __shared__ __align__(16) uint4 tl[4][16 * MR * (WIDE ? RM_XS / 4 : 9)];
   constexpr int LD = 2 * MR;  // 16-byte weight loads per lane and step
@@ -1189,8 +1188,7 @@ __global__ __launch_bounds__(256, 2) void k_bf16_rows_mfma(float *__restrict__ y
 #pragma unroll
     for (int d = 0; d < D; ++d) {
       const int t = tb + d;
-      if (XB == 1) __syncthreads();  // every wave is done with the last step's x
-      float *xw = xs[d % XB];
+      float *xw = xs[d % 2];
       if (64 * NT == 256 || tid < 64 * NT) {
         const uint4 *c = xr[d];
         *reinterpret_cast<uint4 *>(xw + xd) = make_uint4(c[0].x, c[1].x, c[2].x, c[3].x);
@@ -1589,31 +1587,26 @@ static void launch_fp4_t(const GemvArgs *a, int nvec, int pair, hipStream_t st) 
   hipLaunchKernelGGL(k_gemv_fp4_t<NP>, grid, dim3(256), lds, st, *a, pair);
 }
 
-// Row tiles per wave (MR): the pick that leaves the busiest CU the fewest
-// tiles, ceil(workgroups / 256) * MR, and of equals the larger (x staged for
-// more rows) as long as it gives about two workgroups per CU, so that one
-// computes while the other stages. 129280 rows: MR 4, 505 workgroups (64
-// tokens 540 us, MR 1 565); 65536 rows: MR 1 (64 tokens 270 us, MR 4 with 256
-// workgroups 311); 98304 rows, 64 tokens: MR 2, 768 workgroups (393 us, MR 1
-// 406). Up to 16 tokens MR 2 is left out: the weight stream bounds, and more
-// waves keep more of it in flight (98304 rows: MR 1 155 us, MR 2 177).
+// Row tiles per wave: 4 up to 16 tokens, else 2, where that leaves the busiest
+// CU no more tiles than one each (workgroups per CU times tiles) and every CU
+// more than one workgroup, so that one computes while another stages; else 1.
+// Rows of 4096 columns, us with 1 / 4 tiles at 16 tokens: 65536 rows 129 / 145,
+// 98304 185 / 204, 114688 217 / 208, 120000 235 / 212, 129280 245 / 222, 150000
+// 302 / 333; with 1 / 2 at 64 tokens: 57344 348 / 279, 65536 359 / 280, 73728 361 /
+// 392, 90112 431 / 394, 114688 536 / 538, 129280 572 / 543. (2 at 16 tokens and 4
+// beyond gave nothing: 256 and 547 at 129280.) Rows of up to 128 columns are
+// mostly a workgroup's start: the larger tile up to 32 tokens as soon as it fills
+// the CUs (100000 x 64, 16 tokens 13.1 / 10.4, 32 tokens 18.4 / 16.8).
 template <int NT>
 static void launch_rows_mfma_nt(float *y, const float *x, const uint16_t *W, int in, int out,
                                 int round_out, int t0, int n, hipStream_t st) {
-  int mr = 1;
-  long best = (out + 63L) / 64;
-  best = (best + 255) / 256;
-  for (int m = NT == 1 ? 4 : 2; m <= 4; m *= 2) {
-    const long wgs = (out + 64L * m - 1) / (64L * m), cost = (wgs + 255) / 256 * m;
-    if (wgs >= 500 && cost <= best) {
-      best = cost;
-      mr = m;
-    }
-  }
-  auto k = mr == 4 ? k_bf16_rows_mfma<NT, 4, false> : mr == 2 ? k_bf16_rows_mfma<NT, 2, false>
-                                                       : k_bf16_rows_mfma<NT, 1, false>;
-  hipLaunchKernelGGL(k, dim3((unsigned)((out + 64 * mr - 1) / (64 * mr))), dim3(256), 0, st, y, x,
-                     W, in, out, round_out, t0, n, nullptr, nullptr);
+  constexpr int MR = NT == 1 ? 4 : 2;
+  const long one = (out + 63L) / 64, wgs = (out + 64L * MR - 1) / (64L * MR);
+  const bool tiles = wgs > 256 && ((wgs + 255) / 256 * MR <= (one + 255) / 256 ||
+                                   (NT <= 2 && in <= 128));
+  auto k = tiles ? k_bf16_rows_mfma<NT, MR, false> : k_bf16_rows_mfma<NT, 1, false>;
+  hipLaunchKernelGGL(k, dim3((unsigned)(tiles ? wgs : one)), dim3(256), 0, st, y, x, W, in, out,
+                     round_out, t0, n, nullptr, nullptr);
 }
 
 static void launch_rows_mfma(float *y, const float *x, const uint16_t *W, int in, int out,
@@ -1635,18 +1628,19 @@ static void launch_rows_mfma(float *y, const float *x, const uint16_t *W, int in
 // 64-row tiles per CU) favour the tiled form and wide rows or more tokens the
 // matrix unit's (us, tiled / matrix unit). One token: 16384 rows of 128 3.5 / 4.0,
 // of 256 5.3 / 4.7; 40000 of 384 10.0 / 11.5, of 512 15.7 / 13.6; 72000 of 512
-// 20.1 / 21.4, of 4096 163 / 147; 88000 of 4096 171 / 173; 114688 of 4096 176 /
-// 205. Two: 24000 of 192 5.4 / 6.2, of 256 6.7 / 6.6; 96000 of 512 23.8 / 25.2,
-// of 1024 45.2 / 44.2; 100000 of 1024 45.6 / 50.7, of 4096 198 / 195. Three:
+// 20.1 / 21.4, of 4096 163 / 147; 98304 of 1024 40 / 44, of 4096 185 / 166; 106496
+// of 4096 185 / 194; 129280 180 / 210. Two: 24000 of 192 5.4 / 6.2, of 256 6.7 /
+// 6.6; 96000 of 512 23.8 / 25.2, of 1024 45.2 / 44.2; 100000 of 1024 45.6 / 50.7, of
+// 4096 198 / 195; 129280 of 4096 206 / 210. Three:
 // 50000 of 256 8.9 / 10.3; 100000 of 768 38.8 / 39.6, of 1024 53 / 51. Four:
 // 65536 of 192 7.5 / 10, of 256 12.0 / 11.0. Eight: 65536 of 64 4.7 / 7.1, of 128
-// 9.0 / 8.6; 100000 of 128 10.0 / 13.1, of 192 15.9 / 15.9. (16 tokens of 64
-// columns: 8.8 by tiles of four rows a lane, 12.7 here, at 100000 rows; a shape
-// without a use.)
+// 9.0 / 8.6; 100000 of 128 10.0 / 13.1, of 192 15.9 / 15.9. (16 tokens
+// through 100000 x 64 took 8.8 and 32 13.7 with four rows a lane on the VALU,
+// here 10.4 and 16.8; that form lost everywhere else and is gone.)
 static int tiled_width(int n, int out) {
   constexpr int ANY = 0x7fffffff;
   //                             w = 1    2    3    4    5    6     7   more
-  static constexpr int W[5][8] = {{128, 384, 384, 384, 512, ANY, ANY, ANY},   // 1 token
+  static constexpr int W[5][8] = {{128, 384, 384, 384, 512, 1024, ANY, ANY},  // 1 token
                                   {64, 192, 320, 320, 384, 512, 1024, ANY},   // 2
                                   {64, 128, 192, 256, 256, 384, 768, 768},    // 3
                                   {64, 64, 192, 192, 192, 192, 384, 384},     // 4
