@@ -1951,9 +1951,16 @@ int dsv4g_gemv_fp8_float(float *y, const float *x, const uint8_t *W, const float
     return dsv4g_fail(DSV4G_EINVAL, "gemv_fp8_float: bad size");
   // split chains where the row is long, or too ragged for the product chains
   // (2048 rows of 3008 columns 14 us against 17, of 2048 12.6 against 12.0, of
-  // 1024 11 against 7.5; of 2064 12.5 against 22)
+  // 1024 11 against 7.5; of 2064 12.5 against 22), as long as they are the faster
+  // beside a lane per row by these fits (us): the split's rounds of workgroups
+  // against one row's time, which hardly grows with the rows (2048, 4096, 8192,
+  // 32768 rows of 1040 columns, split 10.9, 15.3, 26, 82 and a lane per row 12.2,
+  // 12.1, 12.1, 15; of 4096 16.9, 27, 50, 168 and 39.6, 39.7, 42, 46)
+  const bool xs = mode == 0 && block % 64 == 0;  // k_rowchain's scaled x in LDS
+  const double split = 6 + rows / 1024.0 * (1.5 + 0.9e-3 * in);
+  const double lanes = xs ? 2.9 + 9.0e-3 * in : 2.6 + 11.4e-3 * in;
   if (in % 16 == 0 && (in > PC_MAXIN || (in % 32 && in >= PS_MININ)) && in <= PS_MAXIN &&
-      block % 16 == 0 && ((uintptr_t)x & 15) == 0) {
+      block % 16 == 0 && ((uintptr_t)x & 15) == 0 && split < lanes) {
     // more than the default 64 KB of LDS (a host-side setting of the kernel)
     auto k = mode == 0 ? k_fp8_prodsplit<0> : k_fp8_prodsplit<1>;
     DSV4G_HIP(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -1991,7 +1998,7 @@ int dsv4g_gemv_fp8_float(float *y, const float *x, const uint8_t *W, const float
     a.batch = 1;
     const dim3 grid((rows + 63) / 64);
     const size_t xb = (size_t)in * 4 + (size_t)(64 / block + 2) * ((in + block - 1) / block) * 4;
-    if (mode == 0 && block % 64 == 0)
+    if (xs)
       hipLaunchKernelGGL((k_rowchain<RC_FP8_XS, 1>), grid, dim3(64), xb, (hipStream_t)stream, a);
     else if (mode == 0)
       hipLaunchKernelGGL((k_rowchain<RC_FP8_X, 1>), grid, dim3(64), xb, (hipStream_t)stream, a);

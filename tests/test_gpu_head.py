@@ -260,10 +260,13 @@ def test_bf16_narrow_rows(env, rows, in_, batch):
 
 @pytest.mark.parametrize("rows,in_,block", [(1, 1024, 128), (5, 1040, 16), (130, 4096, 128),
                                             (67, 4080, 32), (33, 2064, 48), (16, 1008, 16),
-                                            (12, 4112, 16)])
+                                            (12, 4112, 16), (2600, 1040, 128), (2700, 1040, 128),
+                                            (3500, 1040, 16), (6600, 4096, 128), (6700, 4096, 128),
+                                            (8300, 4064, 48)])
 def test_fp8_split_rows(env, rows, in_, block):
     """The split product chains (rows of 1024 to 4096 columns, ragged last
-    segments, groups and workgroups, small blocks) and the widths just outside."""
+    segments, groups and workgroups, small blocks), the widths just outside and
+    the numbers of rows from which a lane takes a whole row."""
     orc, lib = env["orc"], env["lib"]
     rng = np.random.default_rng(rows + in_)
     codes = rng.integers(0, 256, (rows, in_)).astype(np.uint8)
