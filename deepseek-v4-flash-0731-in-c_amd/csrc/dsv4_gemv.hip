@@ -1730,6 +1730,39 @@ int dsv4g_launch_gemv_fp4(const GemvArgs *a, int nvec, int nmat, void *stream) {
   return dsv4g_check_launch("gemv_fp4");
 }
 
+// Fits (us) of the two forms of the FP8 projection for several tokens. Matrix
+// unit: up to 8 blocks a row, 1.9 per block for every 512 workgroups (two on a
+// CU), 1.1 for a last 256 (1024 columns: 8192 rows 12.7 to 16 tokens, 18.6 at 33;
+// 32768 rows 19.5, 35, 50 for 16, 32, 33); beyond, four waves share a row tile:
+// 1.15 per block of a wave, then 1.2 for every further 256 workgroups, which are
+// shared out evenly while LDS takes two on a CU (4096 columns: 1024 rows 12, 8192
+// rows 19, 34, 49 for 16, 32, 33 tokens; 8192 columns x 4096 rows 23, 42, 61).
+static double fp8_mfma_us(int rows, int CB, int ks, int nvec, int nmat) {
+  const long wgs = (rows + 64 / ks - 1L) / (64 / ks) * ((nvec + 15) / 16) * nmat;
+  if (ks == 1) {
+    const long last = wgs % 512;
+    const double t = 4.6 + CB * (1.9 * (wgs / 512) + (last > 256 ? 1.9 : last ? 1.1 : 0.0));
+    return std::max(t, 6.0);
+  }
+  const int q = (CB + 3) / 4;
+  const bool two = fp8_mfma_lds<4>(CB) <= 80 * 1024;
+  const double more = two ? std::max(wgs / 256.0 - 1, 0.0) : (double)((wgs + 255) / 256 - 1);
+  return 3.7 + 1.15 * q + 1.2 * q * more;
+}
+
+// VALU: by token and million weights, a row counted to its last lane (a row of
+// 128 columns busies one of its 8 lanes, of 1152 nine of 16, of 2304 18 of 32): 128
+// columns x 512 rows 5.2 and 6.0 for 16 and 33 tokens; 2048 x 4096 7.0, 9.4 for 4, 8;
+// 8192 x 4096 21.7, 29, 51, 96 for 5, 8, 16, 33; four tokens at a time 1024 x 32768
+// 19, 29, 57 for 8, 16, 33, 384 x 32768 9.7 for 4.
+static double fp8_valu_us(int rows, int CB, int sl, bool many, int nvec, int nmat) {
+  const int lanes = (CB + sl - 1) / sl * sl;
+  const double c = sl == 32 ? 0.035 + 0.05 * CB / lanes
+                 : many     ? (sl == 16 ? 0.01 + 0.05 * CB / lanes : 0.035 + 0.0014 * CB)
+                            : (sl == 16 ? 0.062 : 0.055);
+  return 5 + c * 128e-6 * lanes * nvec * nmat * rows;
+}
+
 int dsv4g_launch_gemv_fp8(const GemvArgs *a, int nvec, int nmat, void *stream) {
   if (fp8_shape_ok(a->in, "gemv_fp8")) return DSV4G_EINVAL;
   if (a->rows <= 0 || nvec <= 0) return dsv4g_fail(DSV4G_EINVAL, "gemv_fp8: bad size");
@@ -1746,20 +1779,10 @@ int dsv4g_launch_gemv_fp8(const GemvArgs *a, int nvec, int nmat, void *stream) {
   // (and the four tokens' activations fit LDS beside the rest: in <= 2048)
   const bool many = nvec > 1 && a->in <= 2048 &&
                     (long)(a->rows + 256 / sl - 1) / (256 / sl) * nmat >= 1024;
-  // Several tokens on the matrix unit where it is the faster by these fits (us).
-  // Matrix unit: a round of workgroups costs 1.4 per block of a wave with a CU
-  // each (in > 1024: 4 waves share a row tile: 8192 columns x 4096 rows 24, 46,
-  // 66 for 16, 32, 33 tokens; 4096 x 1024 13), 2.3 with two workgroups on a CU
-  // (1024 x 32768: 20, 41, 56). VALU: 0.083 per token and million weights, 0.052
-  // four tokens at a time (8192 x 4096 rows: 5 tokens 21.7, 8 30.7, 16 52, 33 97;
-  // 1024 x 32768: 8 tokens 19.6, 16 32, 33 63; 4096 x 1024: 16 tokens 11, 33 17).
+  // several tokens on the matrix unit where it is the faster
   if (nvec > 1 && a->in % 128 == 0) {
     const int ks = CB > 8 ? 4 : 1;
-    const long wgs = (a->rows + 64 / ks - 1L) / (64 / ks) * ((nvec + 15) / 16) * nmat;
-    const double mfma = ks == 4 ? 2 + 1.4 * ((CB + 3) / 4) * ((wgs + 255) / 256)
-                                : 2 + 2.3 * CB * ((wgs + 511) / 512);
-    const double valu = 5 + (many ? 0.052 : 0.083) * 1e-6 * nvec * nmat * a->rows * a->in;
-    if (mfma < valu) {
+    if (fp8_mfma_us(a->rows, CB, ks, nvec, nmat) < fp8_valu_us(a->rows, CB, sl, many, nvec, nmat)) {
       DSV4G_TRY(ks == 4 ? launch_fp8_proj_mfma<4>(a, nvec, nmat, st)
                         : launch_fp8_proj_mfma<1>(a, nvec, nmat, st));
       return dsv4g_check_launch("gemv_fp8");

@@ -98,7 +98,10 @@ def test_pair(env):
 
 @pytest.mark.parametrize("rows,cols,n", [(1, 128, 2), (70, 128, 17), (333, 384, 16), (130, 1024, 40),
                                          (1000, 1024, 33), (2100, 1152, 33), (2050, 2048, 33),
-                                         (1040, 8192, 21), (1024, 4096, 23), (1024, 4096, 24)])
+                                         (1040, 8192, 21), (1024, 4096, 22), (1024, 4096, 23),
+                                         (1024, 4096, 24), (2999, 128, 5), (2999, 128, 9),
+                                         (9001, 384, 17), (5003, 1024, 33), (8200, 1024, 23),
+                                         (1201, 8192, 33), (3001, 4736, 18), (2999, 4864, 17)])
 def test_several_tokens(env, rows, cols, n):
     """Both sides of the rule between the VALU's and the matrix unit's chains:
     one to 64 blocks a row, ragged row tiles, workgroups and token groups, a
