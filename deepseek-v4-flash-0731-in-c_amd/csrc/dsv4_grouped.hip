@@ -7,7 +7,9 @@
 //      (the reference's activation quant, exact);
 //   2. router: every logit as the reference's sequential fmaf chain on the
 //      fp32 matrix unit, then the reference's selection and weights - indices
-//      and weights identical to the reference;
+//      and weights identical to the reference (beyond RX_ALL_TOKENS: BF16 MFMA
+//      logits with sum|g*x| for a rigorous error bound, candidate experts per
+//      token, the chains of the candidates only);
 //   3. dispatch: deterministic per-expert position lists (ascending token, as
 //      expert_forward_batch_routes gathers them, src/dsv4/dsv4_model.c:6498-6524)
 //      and a token-tile table (one workgroup up to 1024 routes); the shared
@@ -70,10 +72,13 @@ __device__ __forceinline__ uint32_t scale_code(float s) { return (f2u(s) >> 23) 
 
 // ------------------------------------------------------- batch quant ----
 // The reference activation quant per (token, 128-group), stored as the
-// exact BF16 value of each quantised element (E4M3 grid value x scale); and
+// exact BF16 value of each quantised element (E4M3 grid value x scale); with
+// off_bf16, per 256-column piece of a token a flag: 1 when a value of x in it
+// is not BF16-valued (the router bound then widens), written either way; and
 // zeroes *zero (the route placement's counter) for the kernels after it.
 // 16-byte loads: a half wave per group.
 __global__ __launch_bounds__(256) void k_batch_quant(uint16_t *__restrict__ xb,
+                                                     int *__restrict__ off_bf16,
                                                      int *__restrict__ zero,
                                                      const float *__restrict__ x, int T, int H) {
   if (blockIdx.x == 0 && threadIdx.x == 0) *zero = 0;
@@ -98,19 +103,515 @@ __global__ __launch_bounds__(256) void k_batch_quant(uint16_t *__restrict__ xb,
   const uint32_t h2 = f2u(quant_e4m3(v.z, inv) * scale) >> 16;
   const uint32_t h3 = f2u(quant_e4m3(v.w, inv) * scale) >> 16;
   if (live) *reinterpret_cast<uint2 *>(xb + t * H + c) = make_uint2(h0 | (h1 << 16), h2 | (h3 << 16));
+  if (!off_bf16) return;
+  const bool exact = bf16_round(v.x) == v.x && bf16_round(v.y) == v.y &&
+                     bf16_round(v.z) == v.z && bf16_round(v.w) == v.w;
+  const bool any_off = __any(!exact);
+  if (lane == 0) off_bf16[w] = any_off ? 1 : 0;  // w = t * pieces + c0 / 256
 }
 
 // ---------------------------------------------------------- router ------
+// ---- very many tokens: candidates, and the chains of those only.
+// Approximate logits and sum|g*x| with BF16 MFMA. Tile: 64 tokens x 64
+// experts; wave w takes experts e0+16w..+15 against all 64 tokens. K runs in
+// steps of 128: x (truncated to BF16: exact for BF16-valued inputs) is staged
+// into a double-buffered LDS tile, one barrier per step; each thread's x and
+// gate operands are loaded two steps ahead into a register ring of
+// range-checked loads (rows past T or E read zeros).
+struct RlRegs {
+  uint4 x[8];  // 4 columns (fp32) of tokens 16 w + 2 i + l / 32, i = 0..7
+  uint4 g[4];  // this lane's gate operands of the step's 4 MFMA k-steps
+};
+
+__device__ __forceinline__ void rl_load(RlRegs &R, BufRsrc rx, uint32_t xo, uint32_t xstep,
+                                        BufRsrc rg, uint32_t go, int k0) {
+#pragma unroll
+  for (int i = 0; i < 8; ++i) R.x[i] = buf_load16(rx, xo + i * xstep + 4u * (uint32_t)k0);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) R.g[j] = buf_load16(rg, go + 2u * (uint32_t)(k0 + 32 * j));
+  __builtin_amdgcn_sched_barrier(0);  // issue here, not next to the first use
+}
+
+__device__ __forceinline__ void rl_store(const RlRegs &R, uint16_t *xs, int wv, int l) {
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const uint4 u = R.x[i];
+    *reinterpret_cast<uint2 *>(xs + (16 * wv + 2 * i + l / 32) * 136 + 4 * (l % 32)) =
+        make_uint2((u.x >> 16) | (u.y & 0xFFFF0000u), (u.z >> 16) | (u.w & 0xFFFF0000u));
+  }
+}
+
+__device__ __forceinline__ void rl_mfma(v4f (&acc)[4], v4f (&aab)[4], const RlRegs &R,
+                                        const uint16_t *xs, int l) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const uint4 a = R.g[j];
+    const uint4 aa = make_uint4(a.x & 0x7FFF7FFFu, a.y & 0x7FFF7FFFu, a.z & 0x7FFF7FFFu,
+                                a.w & 0x7FFF7FFFu);
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+      const uint4 b =
+          *reinterpret_cast<const uint4 *>(xs + (16 * f + l % 16) * 136 + 32 * j + 8 * (l / 16));
+      const uint4 bb = make_uint4(b.x & 0x7FFF7FFFu, b.y & 0x7FFF7FFFu, b.z & 0x7FFF7FFFu,
+                                  b.w & 0x7FFF7FFFu);
+      acc[f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
+                                                       __builtin_bit_cast(bf16x8, b), acc[f], 0, 0, 0);
+      aab[f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, aa),
+                                                       __builtin_bit_cast(bf16x8, bb), aab[f], 0, 0, 0);
+    }
+  }
+}
+
+template <int NS>  // H / 128 when known at compile time (fully unrolled K), else 0
+__global__ __launch_bounds__(256) void k_router_logits_mfma(float *__restrict__ z,
+                                                            float *__restrict__ zabs,
+                                                            const float *__restrict__ x,
+                                                            const uint16_t *__restrict__ G,
+                                                            int T, int H, int E) {
+  __shared__ __align__(16) uint16_t xs[2][64 * 136];  // [buf][token][128 + 8 pad] bf16
+  const int t0 = blockIdx.x * 64, e0 = blockIdx.y * 64;
+  const int tid = threadIdx.x, l = tid % 64;
+  const int wv = __builtin_amdgcn_readfirstlane(tid / 64);
+  v4f acc[4], aab[4];
+  for (int f = 0; f < 4; ++f) {
+    acc[f] = (v4f){0.f, 0.f, 0.f, 0.f};
+    aab[f] = (v4f){0.f, 0.f, 0.f, 0.f};
+  }
+  // staging: wave w brings tokens 16 w .. + 15, two 512-byte rows per load
+  // (rows past T lie beyond the range and read zeros)
+  const BufRsrc rx = buf_rsrc(x + (size_t)t0 * H, 4u * (uint32_t)(min(T - t0, 64) * H));
+  const uint32_t xo = 4u * (uint32_t)((16 * wv + l / 32) * H + 4 * (l % 32)), xstep = 8u * H;
+  // one range per wave (a per-lane range would serialise the loads); expert
+  // rows past E lie beyond it and read zeros
+  const int we = e0 + 16 * wv;
+  const uint32_t grange = __builtin_amdgcn_readfirstlane(2u * (uint32_t)(max(min(E - we, 16), 0) * H));
+  const BufRsrc rg = buf_rsrc(G + (size_t)min(we, E - 1) * H, grange);
+  const uint32_t go = 2u * (uint32_t)((l % 16) * H + 8 * (l / 16));
+  RlRegs R[3];
+  rl_load(R[0], rx, xo, xstep, rg, go, 0);
+  rl_load(R[1], rx, xo, xstep, rg, go, 128);
+  rl_store(R[0], xs[0], wv, l);
+  __syncthreads();
+  // step s computes from xs[s & 1] with the gate operands of ring slot s % 3,
+  // stores step s + 1 into the other buffer and loads step s + 2 (loads past
+  // the row end are never used)
+  if constexpr (NS > 0) {
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      if (s + 2 < NS) rl_load(R[(s + 2) % 3], rx, xo, xstep, rg, go, 128 * (s + 2));
+      rl_mfma(acc, aab, R[s % 3], xs[s & 1], l);
+      if (s + 1 < NS) {
+        rl_store(R[(s + 1) % 3], xs[(s + 1) & 1], wv, l);
+        __syncthreads();
+      }
+    }
+  } else {
+    // unrolled by three so that the ring slots are compile-time
+    const int ns = H / 128;  // H % 128 == 0
+    for (int s = 0; s < ns; s += 3) {
+      rl_load(R[2], rx, xo, xstep, rg, go, 128 * (s + 2));
+      rl_mfma(acc, aab, R[0], xs[s & 1], l);
+      if (s + 1 < ns) rl_store(R[1], xs[(s + 1) & 1], wv, l);
+      __syncthreads();
+      if (s + 1 >= ns) break;
+      rl_load(R[0], rx, xo, xstep, rg, go, 128 * (s + 3));
+      rl_mfma(acc, aab, R[1], xs[(s + 1) & 1], l);
+      if (s + 2 < ns) rl_store(R[2], xs[s & 1], wv, l);
+      __syncthreads();
+      if (s + 2 >= ns) break;
+      rl_load(R[1], rx, xo, xstep, rg, go, 128 * (s + 4));
+      rl_mfma(acc, aab, R[2], xs[s & 1], l);
+      if (s + 3 < ns) rl_store(R[0], xs[(s + 1) & 1], wv, l);
+      __syncthreads();
+    }
+  }
+  for (int f = 0; f < 4; ++f) {
+    const int t = t0 + 16 * f + l % 16;
+    if (t >= T) continue;
+    for (int v = 0; v < 4; ++v) {
+      const int e = e0 + 16 * wv + 4 * (l / 16) + v;
+      if (e < E) {
+        z[(size_t)t * E + e] = acc[f][v];
+        zabs[(size_t)t * E + e] = aab[f][v];
+      }
+    }
+  }
+}
+
+__device__ __forceinline__ float gamma_n2(int n) {
+  const double nu = (double)n * 0x1p-24;
+  return (float)(nu / (1.0 - nu));
+}
+
+// One wave per token: approximate choices, the k-th best, and every expert
+// within the rigorous error margin of it -> candidate list (ascending id).
+// z / zabs: the router logits and sum|g*x| [T][E]; off_bf16: k_batch_quant's
+// flags, np per token.
+template <int PER>  // experts per lane: E <= 64 PER
+__global__ __launch_bounds__(256) void k_router_cand(int *__restrict__ cand,
+                                                     int *__restrict__ ncand,
+                                                     const float *__restrict__ z,
+                                                     const float *__restrict__ zabs,
+                                                     const int *__restrict__ off_bf16, int np,
+                                                     const float *__restrict__ bias,
+                                                     const int64_t *__restrict__ tid2eid,
+                                                     const int *__restrict__ token_ids, int T,
+                                                     int H, int E, int K) {
+  const int t = blockIdx.x * 4 + threadIdx.x / 64, l = threadIdx.x % 64;
+  if (t >= T) return;
+  int *ct = cand + (size_t)t * E;
+  if (tid2eid) {
+    if (l < K) ct[l] = (int)tid2eid[(size_t)token_ids[t] * K + l];
+    if (l == 0) ncand[t] = K;
+    return;
+  }
+  // every lane's logits loaded at once (indices clamped into the row, no
+  // branch), then masked past E
+  float ch[PER], zv[PER], av[PER];
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const size_t i = (size_t)t * E + min(l + 64 * j, E - 1);
+    zv[j] = z[i];
+    av[j] = zabs[i];
+  }
+  float amax = 0.0f;
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const int e = l + 64 * j;
+    ch[j] = -__builtin_inff();
+    if (e < E) {
+      const float c = sqrt_softplus(zv[j]) + (bias ? bias[e] : 0.0f);
+      ch[j] = c == c ? c : -__builtin_inff();  // NaN is never selected
+      amax = fmaxf(amax, av[j]);
+    }
+  }
+  amax = wave_max(amax) * 1.001f;
+  // is x of this token BF16-valued (the MFMA logits used its BF16 truncation)?
+  bool off = false;
+  for (int j = l; j < np; j += 64) off |= off_bf16[(size_t)t * np + j] != 0;
+  // any-order summation bound, twice (approximate and sequential), plus what
+  // the truncation of a non-BF16 input drops (below 2^-7 of what it keeps);
+  // |d score/dz| <= 1/2; score slack
+  float bound_z = 2.0f * gamma_n2(H) * amax;
+  if (__any(off)) bound_z += 0x1p-7f * amax;
+  const float delta = 2.0f * (0.5f * bound_z + 1e-5f);
+  unsigned long long used = 0ull;  // bit j: expert l+64j taken
+  float kth = -__builtin_inff();
+  for (int k = 0; k < K; ++k) {
+    // the k-th largest choice: DPP wave maximum, then the lowest index
+    // holding it is taken (no LDS round trips)
+    float m = -__builtin_inff();
+    int mj = -1;
+#pragma unroll
+    for (int j = 0; j < PER; ++j)
+      if (!((used >> j) & 1ull) && ch[j] > m) {
+        m = ch[j];
+        mj = j;
+      }
+    const float wm = wave_max_dpp(m);
+    kth = wm;
+    const int bi = wave_min_dpp(mj >= 0 && m == wm ? l + 64 * mj : 0x7fffffff);
+    if (bi != 0x7fffffff && (bi % 64) == l) used |= 1ull << (bi / 64);
+  }
+  const float thr = cand_threshold(kth, delta);
+  // compaction in ascending id: pass j holds ids 64j .. 64j + 63 in lane
+  // order, and each pass appends after the previous one
+  int base = 0;
+  for (int j = 0; j < PER; ++j) {
+    const int e = l + 64 * j;
+    const bool take = e < E && ch[j] >= thr;
+    const unsigned long long m = __ballot(take);
+    const int before = __popcll(m & ((1ull << l) - 1ull));
+    if (take) ct[base + before] = e;
+    base += __popcll(m);
+  }
+  if (l == 0) ncand[t] = base;
+}
+
+// Exclusive prefix sum of n[0..T) into off[0..T], one workgroup.
+__global__ __launch_bounds__(1024) void k_scan_counts(int *__restrict__ off,
+                                                      const int *__restrict__ n, int T) {
+  // exclusive prefix of n[0, T) into off, off[T] = the total: 4096 counts a
+  // pass, 4 consecutive per thread, a wave scan by shuffles, the 16 wave
+  // totals scanned by wave 0 (two barriers a pass)
+  __shared__ int wsum[16];
+  __shared__ int carry;
+  const int tid = threadIdx.x, lane = tid % 64, wv = tid / 64;
+  if (tid == 0) carry = 0;
+  __syncthreads();
+  for (int b = 0; b < T; b += 4096) {
+    const int i0 = b + 4 * tid;
+    int v[4], run = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      v[j] = i0 + j < T ? n[i0 + j] : 0;
+      run += v[j];
+    }
+    int inc = run;  // inclusive scan of the threads' sums within the wave
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int u = __shfl_up(inc, o, 64);
+      if (lane >= o) inc += u;
+    }
+    if (lane == 63) wsum[wv] = inc;
+    __syncthreads();
+    if (wv == 0) {
+      int ws = lane < 16 ? wsum[lane] : 0;
+#pragma unroll
+      for (int o = 1; o < 16; o <<= 1) {
+        const int u = __shfl_up(ws, o, 64);
+        if (lane >= o) ws += u;
+      }
+      if (lane < 16) wsum[lane] = ws;  // inclusive over waves
+    }
+    __syncthreads();
+    int x = carry + (wv > 0 ? wsum[wv - 1] : 0) + inc - run;  // exclusive at i0
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (i0 + j < T) off[i0 + j] = x;
+      x += v[j];
+    }
+    __syncthreads();  // every thread has read carry and wsum
+    if (tid == 0) carry += wsum[15];
+    __syncthreads();
+  }
+  if (tid == 0) off[T] = carry;
+}
+
+// Exact logits of every candidate: the reference's column-order fmaf chain
+// (src/dsv4/dsv4_model.c:298-303), one lane per (token, candidate). A wave
+// takes 64 consecutive chains (the candidates of a few consecutive tokens).
+// Per 64-column step the wave's 64 gate pieces (128 bytes each) are loaded
+// as whole lines, 8 lanes a row, and staged in the wave's own LDS rows, from
+// which each lane reads its row; x is loaded directly (the lanes of one
+// token share its lines). Both are loaded a step ahead into registers. A
+// lane per chain reading its own row straight from memory touches 64 lines
+// per load instruction, and the L1 cannot hold the rows between uses.
+#define RC_ROW 144          // LDS bytes per staged gate piece (128 + 16: conflict-free row reads)
+#define RC_BAD 0x80000000u  // an offset past the gate matrix (reads zeros)
+__global__ __launch_bounds__(256) void k_router_chains(float *__restrict__ cscore,
+                                                       float *__restrict__ cchoice,
+                                                       const int *__restrict__ cand,
+                                                       const int *__restrict__ chain_off,
+                                                       const float *__restrict__ x,
+                                                       const uint16_t *__restrict__ G,
+                                                       const float *__restrict__ bias, int T,
+                                                       int H, int E) {
+  __shared__ __align__(16) uint8_t gs[4][64 * RC_ROW];
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), l = threadIdx.x % 64;
+  const int total = chain_off[T];
+  const BufRsrc rg = buf_rsrc(G, 2u * (uint32_t)E * (uint32_t)H);
+  uint8_t *buf = gs[wv];
+  const int nst = H / 64;  // H % 128 == 0
+  for (int g0 = (blockIdx.x * 4 + wv) * 64; g0 < total; g0 += gridDim.x * 256) {
+    const int g = g0 + l;
+    int t = 0, c = 0, e = -1;
+    if (g < total) {
+      int lo = 0, hi = T;  // chain_off[lo] <= g < chain_off[lo+1]
+      while (hi - lo > 1) {
+        const int mid = (lo + hi) / 2;
+        if (chain_off[mid] <= g) lo = mid;
+        else hi = mid;
+      }
+      t = lo;
+      c = g - chain_off[t];
+      e = cand[(size_t)t * E + c];
+      if (e < 0 || e >= E) e = -1;
+    }
+    // staging: load k brings piece l % 8 of chain 8 k + l / 8's row
+    uint32_t srow[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int ek = __shfl(e, 8 * k + l / 8, 64);
+      srow[k] = ek >= 0 ? 2u * (uint32_t)ek * (uint32_t)H + 16u * (l % 8) : RC_BAD;
+    }
+    auto goff = [&](int k, int st) { return srow[k] == RC_BAD ? RC_BAD : srow[k] + 128u * st; };
+    const float *xr = x + (size_t)t * H;
+    uint4 gv[8];
+    float4 xv[16];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) gv[k] = buf_load16(rg, goff(k, 0));
+#pragma unroll
+    for (int i = 0; i < 16; ++i) xv[i] = *reinterpret_cast<const float4 *>(xr + 4 * i);
+    float acc = 0.0f;
+    for (int st = 0; st < nst; ++st) {
+      // the wave's LDS operations run in order: these writes follow the
+      // previous step's reads and precede this step's
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+        *reinterpret_cast<uint4 *>(buf + (8 * k + l / 8) * RC_ROW + 16 * (l % 8)) = gv[k];
+      float4 xc[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) xc[i] = xv[i];
+      if (st + 1 < nst) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) gv[k] = buf_load16(rg, goff(k, st + 1));
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          xv[i] = *reinterpret_cast<const float4 *>(xr + 64 * (st + 1) + 4 * i);
+      }
+      const uint8_t *mine = buf + l * RC_ROW;
+#pragma unroll
+      for (int cc = 0; cc < 8; ++cc) {
+        const uint4 w = *reinterpret_cast<const uint4 *>(mine + 16 * cc);
+        const float4 xa = xc[2 * cc], xb = xc[2 * cc + 1];
+        acc = fmaf(u2f(w.x << 16), xa.x, acc);
+        acc = fmaf(u2f(w.x & 0xFFFF0000u), xa.y, acc);
+        acc = fmaf(u2f(w.y << 16), xa.z, acc);
+        acc = fmaf(u2f(w.y & 0xFFFF0000u), xa.w, acc);
+        acc = fmaf(u2f(w.z << 16), xb.x, acc);
+        acc = fmaf(u2f(w.z & 0xFFFF0000u), xb.y, acc);
+        acc = fmaf(u2f(w.w << 16), xb.z, acc);
+        acc = fmaf(u2f(w.w & 0xFFFF0000u), xb.w, acc);
+      }
+    }
+    if (g < total) {
+      float sc = 0.0f, ch = -__builtin_inff();
+      if (e >= 0) {
+        sc = sqrt_softplus(acc);
+        ch = sc + (bias ? bias[e] : 0.0f);
+      }
+      cscore[(size_t)t * E + c] = sc;
+      cchoice[(size_t)t * E + c] = ch;
+    }
+  }
+}
+
+
+// k_router_chains with x staged in LDS: a wave's 64 consecutive chains
+// belong to at most 63 / K + 2 tokens (every token has at least K
+// candidates), at most RCX_TOK for K >= 5, so per 64-column step the wave
+// stages those tokens' x slices (16-byte pieces, 4 per lane) beside its
+// gate pieces in its own LDS rows, and registers carry both RCX_DEPTH steps
+// ahead (a one-step read-ahead left each step waiting a memory round trip;
+// the x slice per lane alone took 64 VGPRs a step). Loads of steps past the
+// row are range-checked and never used; no load sits under a branch. Same
+// chains, same column order, same outputs.
+#define RCX_TOK 16
+#define RCX_DEPTH 4
+#define RCX_XROW (64 * 4 + 16)  // LDS bytes per staged x slice
+__global__ __launch_bounds__(256) void k_router_chains_x(float *__restrict__ cscore,
+                                                         float *__restrict__ cchoice,
+                                                         const int *__restrict__ cand,
+                                                         const int *__restrict__ chain_off,
+                                                         const float *__restrict__ x,
+                                                         const uint16_t *__restrict__ G,
+                                                         const float *__restrict__ bias, int T,
+                                                         int H, int E) {
+  __shared__ __align__(16) uint8_t gs[4][64 * RC_ROW];
+  __shared__ __align__(16) uint8_t xsh[4][RCX_TOK * RCX_XROW];
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), l = threadIdx.x % 64;
+  const int total = chain_off[T];
+  const BufRsrc rg = buf_rsrc(G, 2u * (uint32_t)E * (uint32_t)H);
+  uint8_t *gbuf = gs[wv], *xbuf = xsh[wv];
+  const int nst = H / 64;  // H % 128 == 0
+  for (int g0 = (blockIdx.x * 4 + wv) * 64; g0 < total; g0 += gridDim.x * 256) {
+    const int g = g0 + l;
+    int t = 0, c = 0, e = -1;
+    if (g < total) {
+      int lo = 0, hi = T;  // chain_off[lo] <= g < chain_off[lo+1]
+      while (hi - lo > 1) {
+        const int mid = (lo + hi) / 2;
+        if (chain_off[mid] <= g) lo = mid;
+        else hi = mid;
+      }
+      t = lo;
+      c = g - chain_off[t];
+      e = cand[(size_t)t * E + c];
+      if (e < 0 || e >= E) e = -1;
+    }
+    const int tf = __builtin_amdgcn_readfirstlane(t);  // lane 0's chain is live
+    const int tt = min(max(t - tf, 0), RCX_TOK - 1);
+    uint32_t srow[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int ek = __shfl(e, 8 * k + l / 8, 64);
+      srow[k] = ek >= 0 ? 2u * (uint32_t)ek * (uint32_t)H + 16u * (l % 8) : RC_BAD;
+    }
+    // x of tokens tf .. tf + RCX_TOK - 1 (rows past T read zeros); piece
+    // p = l + 64 i: token p / 16, columns 4 (p % 16) of the step
+    const BufRsrc rx = buf_rsrc(x + (size_t)tf * H, 4u * (uint32_t)min(T - tf, RCX_TOK) * (uint32_t)H);
+    auto gload = [&](uint4 (&gv)[8], int st) {
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+        gv[k] = buf_load16(rg, srow[k] == RC_BAD ? RC_BAD : srow[k] + 128u * st);
+    };
+    auto xload = [&](uint4 (&xq)[4], int st) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int p = l + 64 * i;
+        xq[i] = buf_load16(rx, 4u * ((uint32_t)(p / 16) * (uint32_t)H + 64u * st + 4u * (p % 16)));
+      }
+    };
+    uint4 gv[RCX_DEPTH][8], xq[RCX_DEPTH][4];
+#pragma unroll
+    for (int d = 0; d < RCX_DEPTH; ++d) {
+      gload(gv[d], d);
+      xload(xq[d], d);
+    }
+    float acc = 0.0f;
+    int s0 = 0;
+    do {
+#pragma unroll
+      for (int d = 0; d < RCX_DEPTH; ++d) {
+        const int st = s0 + d;
+        // the wave's LDS operations run in order: these writes follow the
+        // previous step's reads and precede this step's
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+          *reinterpret_cast<uint4 *>(gbuf + (8 * k + l / 8) * RC_ROW + 16 * (l % 8)) = gv[d][k];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int p = l + 64 * i;
+          *reinterpret_cast<uint4 *>(xbuf + (p / 16) * RCX_XROW + 16 * (p % 16)) = xq[d][i];
+        }
+        gload(gv[d], st + RCX_DEPTH);
+        xload(xq[d], st + RCX_DEPTH);
+        if (st < nst) {
+          const uint8_t *mine = gbuf + l * RC_ROW;
+          const float4 *xr = reinterpret_cast<const float4 *>(xbuf + tt * RCX_XROW);
+#pragma unroll
+          for (int cc = 0; cc < 8; ++cc) {
+            const uint4 w = *reinterpret_cast<const uint4 *>(mine + 16 * cc);
+            const float4 xa = xr[2 * cc], xb = xr[2 * cc + 1];
+            acc = fmaf(u2f(w.x << 16), xa.x, acc);
+            acc = fmaf(u2f(w.x & 0xFFFF0000u), xa.y, acc);
+            acc = fmaf(u2f(w.y << 16), xa.z, acc);
+            acc = fmaf(u2f(w.y & 0xFFFF0000u), xa.w, acc);
+            acc = fmaf(u2f(w.z << 16), xb.x, acc);
+            acc = fmaf(u2f(w.z & 0xFFFF0000u), xb.y, acc);
+            acc = fmaf(u2f(w.w << 16), xb.z, acc);
+            acc = fmaf(u2f(w.w & 0xFFFF0000u), xb.w, acc);
+          }
+        }
+      }
+      s0 += RCX_DEPTH;
+    } while (s0 < nst);
+    if (g < total) {
+      float sc = 0.0f, ch = -__builtin_inff();
+      if (e >= 0) {
+        sc = sqrt_softplus(acc);
+        ch = sc + (bias ? bias[e] : 0.0f);
+      }
+      cscore[(size_t)t * E + c] = sc;
+      cchoice[(size_t)t * E + c] = ch;
+    }
+  }
+}
+
+// ---- the selection.
 // The routes of one token (one wave; lane k carries route k in selection
-// order): the reference selection (src/dsv4/dsv4_model.c:6866-6906) over the
-// E experts' choices cc[i], strict '>' in ascending id so the lowest id wins a
-// tie; weights from the unbiased scores cs[i]; then an exchange sort by id.
-// Hash layers take the token's tid2eid experts in table order (hash_e: lane
-// k's expert, -1 past K; an expert outside [0, E) scores 0). PER: experts per
-// lane (E <= 64 PER).
+// order): the reference selection (src/dsv4/dsv4_model.c:6866-6906) over nc
+// scored choices cc[i] of experts ct[i] (ct null: expert i, all of them),
+// strict '>' in ascending position so the lowest id wins a tie; weights from
+// the unbiased scores cs[i]; then an exchange sort by id. Hash layers take
+// the token's tid2eid experts in table order (hash_e: lane k's expert, -1
+// past K) with cs indexed by route (ct given) or by expert (ct null; an
+// expert outside [0, E) scores 0). PER: choices per lane (nc <= 64 PER).
 template <int PER>
 __device__ __forceinline__ void router_finalize_wave(int l, int *__restrict__ idx,
                                                      float *__restrict__ wt,
+                                                     const int *__restrict__ ct, int nc,
                                                      const float *__restrict__ cs,
                                                      const float *__restrict__ cc, bool hash,
                                                      int hash_e, int E, int K,
@@ -120,18 +621,20 @@ __device__ __forceinline__ void router_finalize_wave(int l, int *__restrict__ id
   if (hash) {
     if (l < K) {
       my_e = hash_e;
-      my_sc = my_e >= 0 && my_e < E ? cs[my_e] : 0.0f;
+      my_sc = ct ? cs[l] : (my_e >= 0 && my_e < E ? cs[my_e] : 0.0f);
     }
   } else {
-    // choices and scores all loaded up front (a score fetched per route would
-    // be a dependent memory round trip per route)
+    // choices, scores and ids all loaded up front (a score or id fetched
+    // per route would be a dependent memory round trip per route)
     float v[PER], sv[PER];
+    int ev[PER];
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
       const int i = l + 64 * j;
-      const float c = i < E ? cc[i] : -__builtin_inff();
+      const float c = i < nc ? cc[i] : -__builtin_inff();
       v[j] = c == c ? c : -__builtin_inff();  // NaN is never selected
-      sv[j] = i < E ? cs[i] : 0.0f;
+      sv[j] = i < nc ? cs[i] : 0.0f;
+      ev[j] = ct && i < nc ? ct[i] : i;
     }
     for (int k = 0; k < K; ++k) {
       // the largest choice, the lowest index among equals (the reference's
@@ -149,17 +652,22 @@ __device__ __forceinline__ void router_finalize_wave(int l, int *__restrict__ id
       const int bi = wave_min_dpp(mj >= 0 && m == wm ? l + 64 * mj : 0x7fffffff);
       // bi is wave-uniform: its slot j, then the value from its lane
       float bs = 0.0f;
+      int be = 0;
 #pragma unroll
       for (int j = 0; j < PER; ++j)
-        if (j == bi / 64) bs = sv[j];
+        if (j == bi / 64) {
+          bs = sv[j];
+          be = ev[j];
+        }
       bs = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(bs), bi % 64));
+      be = __builtin_amdgcn_readlane(be, bi % 64);
       if (bi % 64 == l) {
 #pragma unroll
         for (int j = 0; j < PER; ++j)
           if (j == bi / 64) v[j] = -__builtin_inff();  // taken
       }
       if (l == k) {
-        my_e = bi;
+        my_e = be;
         my_sc = bs;
       }
     }
@@ -180,6 +688,19 @@ __device__ __forceinline__ void router_finalize_wave(int l, int *__restrict__ id
     idx[rank] = my_e;
     wt[rank] = my_w;
   }
+}
+
+// Candidate form: the chains of k_router_chains.
+__global__ __launch_bounds__(256) void k_router_finalize(
+    int *__restrict__ idx, float *__restrict__ wt, const int *__restrict__ cand,
+    const int *__restrict__ ncand, const float *__restrict__ cscore,
+    const float *__restrict__ cchoice, int hash, int T, int E, int K, float route_scale) {
+  const int t = blockIdx.x * 4 + threadIdx.x / 64, l = threadIdx.x % 64;
+  if (t >= T) return;
+  const size_t r = (size_t)t * E;
+  router_finalize_wave<16>(l, idx + (size_t)t * K, wt + (size_t)t * K, cand + r, ncand[t],
+                           cscore + r, cchoice + r, hash != 0, l < K ? cand[r + l] : -1, E, K,
+                           route_scale);
 }
 
 // ---- few tokens: the chains on the VALU.
@@ -303,8 +824,7 @@ __global__ __launch_bounds__(64) void k_router_exact(float *__restrict__ cscore,
 }
 
 // One wave per token over every expert's exact score (k_router_exact or
-// dsv4g_launch_router_scores); hash
-// layers take the token's tid2eid experts.
+// dsv4g_launch_router_scores); hash layers take the token's tid2eid experts.
 template <int PER>  // experts per lane: E <= 64 PER
 __global__ __launch_bounds__(256) void k_router_select(
     int *__restrict__ idx, float *__restrict__ wt, const float *__restrict__ cscore,
@@ -314,7 +834,7 @@ __global__ __launch_bounds__(256) void k_router_select(
   if (t >= T) return;
   const size_t r = (size_t)t * E;
   const int he = tid2eid && l < K ? (int)tid2eid[(size_t)token_ids[t] * K + l] : -1;
-  router_finalize_wave<PER>(l, idx + (size_t)t * K, wt + (size_t)t * K, cscore + r,
+  router_finalize_wave<PER>(l, idx + (size_t)t * K, wt + (size_t)t * K, nullptr, E, cscore + r,
                             cchoice + r, tid2eid != nullptr, he, E, K, route_scale);
 }
 
@@ -463,7 +983,7 @@ __global__ __launch_bounds__(1024) void k_select_dispatch(
     if (t < T) {
       const size_t r = (size_t)t * E;
       const int he = tid2eid && l < K ? (int)tid2eid[(size_t)token_ids[t] * K + l] : -1;
-      router_finalize_wave<PER>(l, es + t % SD_WAVES * K, wsel + t % SD_WAVES * K,
+      router_finalize_wave<PER>(l, es + t % SD_WAVES * K, wsel + t % SD_WAVES * K, nullptr, E,
                                 cscore + r, cchoice + r, tid2eid != nullptr, he, E, K,
                                 route_scale);
       if (l < K) {
@@ -1394,7 +1914,8 @@ using namespace dsv4;
 namespace {
 struct BatchWs {
   uint16_t *xb, *yb;
-  float *cscore, *cchoice, *wt, *pos_wt;
+  float *z, *zabs, *cscore, *cchoice, *wt, *pos_wt;
+  int *off_bf16, *cand, *ncand, *chain_off;  // with z, zabs: beyond RX_ALL_TOKENS
   int *rcnt, *idx, *counts, *bh, *pos_off, *tile_off, *pos_token, *pos_route;
   uint16_t *ro;
   size_t bytes;
@@ -1436,6 +1957,11 @@ int side_stream(hipStream_t st, SideStream **out) {
 // us, 128 27.8, 256 41), beyond on the fp32 matrix unit (38 us from 16 tokens
 // on, 38 at 256, 47 at 777).
 #define RX_MAX_TOKENS 192
+// Beyond this many the chains of the candidates only: every expert's chains
+// compete with the shared expert's GEMMs beside them for the matrix unit (layer
+// us, all experts / candidates: 2500 tokens 1478 / 1496, 3000 1656 / 1664, 3500
+// 1825 / 1826, 4096 2035 / 2012, 8192 3577 / 3560).
+#define RX_ALL_TOKENS 3400
 // Up to this many tokens the shared expert's tiles are folded into the
 // routed GEMM launches (one stream); beyond, they run on a second stream.
 #define FOLD_MAX_TOKENS 256
@@ -1455,6 +1981,14 @@ BatchWs batch_ws_layout(const DSV4GLayer *L, int T, void *base) {
   };
   w.xb = (uint16_t *)take(t * H * 2);
   w.rcnt = (int *)take(4);
+  if (T > RX_ALL_TOKENS) {
+    w.off_bf16 = (int *)take(t * ((H + 255) / 256) * 4);
+    w.z = (float *)take(t * E * 4);
+    w.zabs = (float *)take(t * E * 4);
+    w.cand = (int *)take(t * E * 4);
+    w.ncand = (int *)take(t * 4);
+    w.chain_off = (int *)take((t + 1) * 4);
+  }
   w.cscore = (float *)take(t * E * 4);
   w.cchoice = (float *)take(t * E * 4);
   w.idx = (int *)take(t * K * 4);
@@ -1513,11 +2047,12 @@ int dsv4g_moe_forward_batch_routes(float *out, const float *x, const DSV4GLayer 
   if (idx_out) w.idx = idx_out;
   if (wt_out) w.wt = wt_out;
 
-  // 1. activation quant (+ BF16-valued flags)
+  const bool all = T <= RX_ALL_TOKENS;  // every expert's chain
+  // 1. activation quant (+ BF16-valued flags for the candidates' bound)
   {
     const size_t waves = (size_t)T * ((H + 255) / 256);
     hipLaunchKernelGGL(k_batch_quant, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, st, w.xb,
-                       w.rcnt, x, T, H);
+                       w.off_bf16, w.rcnt, x, T, H);
   }
   DSV4G_TRY(dsv4g_check_launch("batch_quant"));
   GroupedArgs g = {};
@@ -1618,15 +2153,42 @@ int dsv4g_moe_forward_batch_routes(float *out, const float *x, const DSV4GLayer 
     DSV4G_TRY(dsv4g_check_launch("grouped_down_shared"));
   }
   if (side) DSV4G_HIP(hipEventRecord(side->join, sst));
-  // 2. router: every score exact, then the selection (up to 1024 routes it
-  // shares a launch with the placement)
-  if (T <= RX_MAX_TOKENS)
+  // 2. router: every score exact, or those of the candidates, then the
+  // selection (up to 1024 routes it shares a launch with the placement)
+  if (T <= RX_MAX_TOKENS) {
     hipLaunchKernelGGL(k_router_exact, dim3((unsigned)((T + RX_TOK - 1) / RX_TOK),
                                             (unsigned)((E + RX_EXP - 1) / RX_EXP)),
                        dim3(64), 0, st, w.cscore, w.cchoice, x, L->gate_w, L->bias, T, H, E);
-  else
+  } else if (all) {
     DSV4G_TRY(dsv4g_launch_router_scores(w.cscore, w.cchoice, x, L->gate_w, L->bias, T, H, E, st));
-  if (T * K > 1024) {
+  } else {
+    const dim3 grid((T + 63) / 64, (E + 63) / 64);
+    if (H == 4096)
+      hipLaunchKernelGGL(k_router_logits_mfma<32>, grid, dim3(256), 0, st, w.z, w.zabs, x,
+                         L->gate_w, T, H, E);
+    else
+      hipLaunchKernelGGL(k_router_logits_mfma<0>, grid, dim3(256), 0, st, w.z, w.zabs, x,
+                         L->gate_w, T, H, E);
+    auto cand = E <= 64 ? k_router_cand<1> : E <= 128 ? k_router_cand<2> : E <= 256 ? k_router_cand<4>
+              : E <= 512 ? k_router_cand<8> : k_router_cand<16>;
+    hipLaunchKernelGGL(cand, dim3((T + 3) / 4), dim3(256), 0, st, w.cand, w.ncand, w.z, w.zabs,
+                       w.off_bf16, (H + 255) / 256, L->bias, L->tid2eid, token_ids, T, H, E, K);
+    hipLaunchKernelGGL(k_scan_counts, dim3(1), dim3(1024), 0, st, w.chain_off, w.ncand, T);
+    const long bound = (long)T * (K + 4);
+    const int blocks = (int)((bound + 255) / 256 < 4096 ? (bound + 255) / 256 : 4096);
+    // every token has at least K candidates: for K >= 5 a wave's 64 chains
+    // span at most 14 tokens, whose x slices k_router_chains_x stages in LDS
+    if (K >= 5)
+      hipLaunchKernelGGL(k_router_chains_x, dim3(blocks), dim3(256), 0, st, w.cscore, w.cchoice,
+                         w.cand, w.chain_off, x, L->gate_w, L->bias, T, H, E);
+    else
+      hipLaunchKernelGGL(k_router_chains, dim3(blocks), dim3(256), 0, st, w.cscore, w.cchoice,
+                         w.cand, w.chain_off, x, L->gate_w, L->bias, T, H, E);
+    hipLaunchKernelGGL(k_router_finalize, dim3((T + 3) / 4), dim3(256), 0, st, w.idx, w.wt,
+                       w.cand, w.ncand, w.cscore, w.cchoice, L->tid2eid ? 1 : 0, T, E, K,
+                       L->route_scale);
+  }
+  if (all && T * K > 1024) {
     auto sel = E <= 64 ? k_router_select<1> : E <= 128 ? k_router_select<2>
              : E <= 256 ? k_router_select<4> : E <= 512 ? k_router_select<8>
                         : k_router_select<16>;
