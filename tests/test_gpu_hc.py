@@ -278,17 +278,48 @@ def test_hc_pre_split_chains(env, mult, hid, n):
         assert same_bits(b[t], orc.rmsnorm_bf16(ob[None], norm, 1e-6, 1)[0]), t
 
 
+def hc_split_scales(orc, S, fn, base):
+    """Scales for mult 4 (powers of two) with which post's arguments are about
+    -12, where the sigmoid passes a relative change on, and the others' about 3 in
+    magnitude, so that a chain off by its last place shows in post or comb: checked
+    here on at least half of the 20 mixes that those depend on. fn's post rows are
+    negated where their sums are positive."""
+    K = S.size
+    acc = np.zeros(24, np.float32)
+    for k in range(K):  # the chains, to a rare double rounding
+        acc = (fn[:, k].astype(np.float64) * np.float64(S[k]) + acc).astype(np.float32)
+    flip = np.flatnonzero(acc[4:8] > 0) + 4
+    fn[flip] *= -1
+    acc[flip] *= -1
+    rs = np.float32(1 / np.sqrt(np.mean(S.astype(np.float64) ** 2) + 1e-6))
+    mix = np.abs(acc.astype(np.float64) * rs)
+    size = [float(np.median(mix[i])) for i in (slice(0, 4), slice(4, 8), slice(8, 24))]
+    sc = np.array([2.0 ** np.clip(np.round(np.log2(t / m)), -126, 127) if m > 0 else 2.0 ** 120
+                   for m, t in zip(size, (3, 12, 3))], np.float32)
+
+    def outputs(a):
+        _, post, comb = orc.hc_split((a * rs).astype(np.float32), sc, base, 4, 20, 1e-6)
+        return post.tobytes() + comb.tobytes()
+    was, seen = outputs(acc), 0
+    for i in range(4, 24):
+        a = acc.copy()
+        a[i] = np.nextafter(a[i], np.float32(-np.inf)) if a[i] else np.float32(2.0 ** -126)
+        seen += outputs(a) != was
+    assert seen >= 10, seen
+    return sc
+
+
 @pytest.mark.parametrize("kind", ["zeros", "growing", "ones", "cancelling", "power_of_two",
                                   "tiny", "subnormal", "huge", "steps", "zero_crossings", "sparse",
-                                  "overflow"])
+                                  "overflow", "infinite"])
 def test_hc_pre_split_chain_values(env, kind):
     """Sums whose segments do not follow from their guesses: exact zeros, sums
     that double from segment to segment, ties at every step, sums that return
-    to zero, that stay at a power of two, subnormal and overflowing sums, and
+    to zero, that stay at a power of two, subnormal, huge and infinite sums, and
     sums just inside the fp32 range whose guesses overflow (terms that the chain
-    loses, then one that takes only the guess past it; both signs). The
-    mixes reach the outputs through post and comb (scale 1, base 0; where they
-    are near 2^128, scale 2^-126)."""
+    loses, then one that takes only the guess past it; both signs). The mixes
+    reach the outputs through post and comb, with a scale at which one last
+    place of a chain shows there (hc_split_scales)."""
     orc, lib = env["orc"], env["lib"]
     mult, hid = 4, 4096
     K, mix_n = mult * hid, 24
@@ -332,12 +363,13 @@ def test_hc_pre_split_chain_values(env, kind):
         fn[:, 0], fn[:, 1:600] = 1.5 * 2.0 ** 126, 0.4 * 2.0 ** 103
         fn[:, K - 20] = 2.0 ** 127 + 2.0 ** 125 - 2.0 ** 110
         fn[::2] *= -1
+    elif kind == "infinite":  # post's sums alone: comb's would be NaN
+        fn[4:8] = 2.0 ** 125
     else:
         S[rng.random(K) < 0.99] = 0
     S, fn = S.astype(np.float32), fn.astype(np.float32)
-    sc, base = np.ones(3, np.float32), np.zeros(mix_n, np.float32)
-    if kind == "overflow":
-        sc[:] = 2.0 ** -126
+    base = np.zeros(mix_n, np.float32)
+    sc = hc_split_scales(orc, S, fn, base)
     b, p, c = (H(v) for v in lib.hc_pre(T(env, S[None]), T(env, fn), T(env, sc), T(env, base),
                                         mult))
     ob, op, oc = orc.hc_pre(S, fn, sc, base, mult)

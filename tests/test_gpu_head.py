@@ -283,13 +283,13 @@ def test_fp8_split_rows(env, rows, in_, block):
 
 @pytest.mark.parametrize("kind", ["zeros", "growing", "ones", "cancelling", "power_of_two",
                                   "subnormal", "huge", "steps", "ties", "sparse",
-                                  "overflow"])
+                                  "overflow", "infinite"])
 def test_fp8_split_values(env, kind):
     """Sums whose segments do not follow from their guesses (as
     test_hc_pre_split_chain_values): every row bit-exact. "overflow": the first
     product, then terms below half a step that the chain loses and a guess
     counts, then one that takes the guess past the fp32 range and the chain
-    just below it, in both signs."""
+    just below it, in both signs; "infinite": sums that leave it."""
     orc, lib = env["orc"], env["lib"]
     rows, in_ = 12, 4096
     rng = np.random.default_rng(23)
@@ -324,10 +324,13 @@ def test_fp8_split_values(env, kind):
         x[:] = 0
         x[0], x[1:600] = 1.5 * 2.0 ** 126, 0.4 * 2.0 ** 103
         x[in_ - 20] = 2.0 ** 127 + 2.0 ** 125 - 2.0 ** 110
+    elif kind == "infinite":
+        x[:] = np.where(k % 900 < 450, 2.0 ** 122, -2.0 ** 122)
+        x[k > 3000] = 2.0 ** 126
     else:
         x[rng.random(in_) < 0.98] = 0
     codes, scales = orc.quant_fp8_blocks_absmax(w.astype(np.float32))
-    if kind in ("power_of_two", "ties", "overflow"):
+    if kind in ("power_of_two", "ties", "overflow", "infinite"):
         scales[:] = 1.0 / 448.0 * 448.0
         codes[:] = 0x38  # 1.0
     if kind == "overflow":
