@@ -904,7 +904,8 @@ __global__ __launch_bounds__(256) void k_fp8_prodchain(float *__restrict__ y,
 // steps serves them all. Bound: instruction issue of the candidates' chains
 // (12 per column and segment, on segments as long as the longest of the wave's,
 // about 1.7 times the mean), then the serial walk and the first memory round
-// trip; 2048 x 4096: 15.1 us, 20.9 us as one add chain per row.
+// trip; 2048 x 4096: 15.0 us, 21.0 us as one add chain per row; 50 us where every
+// segment misses (each pair of products all but cancelling).
 #define PS_ROWS 4
 #define PS_MININ 1024
 #define PS_MAXIN 4096  // 64 segments of 64 columns
@@ -1287,8 +1288,9 @@ __global__ __launch_bounds__(256, 2) void k_bf16_rows_mfma(float *__restrict__ y
 // its own row's 64 columns. Two tiles are in flight while one is chained; x
 // enters each fmaf as a scalar operand. LDS holds one tile: the wave's LDS
 // accesses run in order, and the empty asms keep the compiler from moving them
-// across each other. in a multiple of 64; tokens [t0, t0 + TB)
-// present. 129280 x 4096: 185 us, 2 tokens 223.
+// across each other. in a multiple of 64; tokens [t0, t0 + TB) present. 129280 x
+// 4096: 180 to 187 us, and 220 where the matrix lies badly in memory (one
+// allocation in ten, the same each time it is read); 2 tokens 206.
 #define RT_DEPTH 2
 template <int TB>
 __global__ __launch_bounds__(64) void k_bf16_rows_tiled(float *__restrict__ y,
@@ -1651,8 +1653,8 @@ static int tiled_width(int n, int out) {
 
 // Every (token, expert) score and choice of the batched router, [T][E], exact.
 // Token tiles per wave: the fewest with at most one workgroup per CU (256
-// experts: 38 us up to 400 tokens, 47 at 777, 77 at 2048, 119 at 4096 beside
-// the shared expert's GEMMs).
+// experts, beside the shared expert's GEMMs: 53 us at 300 tokens, 61 at 777, 92 at
+// 2048, 143 at 3400; 44, 54, 80 and 121 at the least).
 int dsv4g_launch_router_scores(float *score, float *choice, const float *x, const uint16_t *G,
                                const float *bias, int T, int H, int E, hipStream_t st) {
   const int egroups = (E + 63) / 64;

@@ -1954,8 +1954,8 @@ int side_stream(hipStream_t st, SideStream **out) {
 }
 
 // Up to this many tokens the router's chains run on the VALU (64 tokens 22.8
-// us, 128 27.8, 256 41), beyond on the fp32 matrix unit (38 us from 16 tokens
-// on, 38 at 256, 47 at 777).
+// us, 128 27.8, 256 41), beyond on the fp32 matrix unit (38 us from 16 to 256
+// tokens with the GPU to itself).
 #define RX_MAX_TOKENS 192
 // Beyond this many the chains of the candidates only: every expert's chains
 // compete with the shared expert's GEMMs beside them for the matrix unit (layer

@@ -442,11 +442,14 @@ __global__ void __launch_bounds__(64 * NW) k_hc_pre(HcArgs a) {
 //  - Eight segments compose to one the same way (128 lanes, all 8 candidates
 //    of 16 such), so the serial walk has 16 steps; one whose conditions fail is
 //    walked segment by segment.
-// A workgroup per mix and token: 24 CUs share what one wave of one CU did (83
+// A workgroup per mix and token: 24 CUs share what one wave of one CU did (79
 // us for one token; its chain of 16384 dependent fmaf runs at 10.5 clocks a
 // step). Bound now: launch, one round trip of the row and the state (128 KB
-// per workgroup), then instruction issue of the 4 chain waves. The mix goes to
-// bin's row of the token, where k_hc_finish reads it.
+// per workgroup), then instruction issue of the 4 chain waves; one token 29 us
+// with k_hc_finish. Where every segment misses (each pair of products cancelling
+// but for the roundings) the reruns add a chain of their own per round of
+// workgroups: 133 us at one token, 495 at 40. The mix goes to bin's row of the
+// token, where k_hc_finish reads it.
 constexpr int SP_T = 1024;         // threads, and 16-column pieces at most
 constexpr int SP_SEG = 128;        // segments: 8 pieces each (fewer for a shorter row)
 constexpr int SP_MAXK = 16 * SP_T;
@@ -638,7 +641,7 @@ __global__ void __launch_bounds__(SP_T) k_hc_mix_split(float *__restrict__ bin,
 // column c % 4 = lane / 16 of 16 columns back with one 16-byte read, the next
 // step's while this step's 16 MFMAs run. LDS operations of the one wave are in
 // order, so it needs no barrier. Measured 82 us up to 300 tokens, 88 at 777,
-// 105 at 4096 (with k_hc_finish 113 us at 777 tokens; 320 us as one workgroup of
+// 105 at 4096 (with k_hc_finish 106 us at 777 tokens; 313 us as one workgroup of
 // chains per token in four rounds).
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 constexpr int MX_D = 4;    // steps of loads in flight
@@ -933,7 +936,7 @@ bool overlap(const float *a, size_t na, const float *b, size_t nb) {
 }
 
 // Up to this many tokens hc_pre's chains are split over a workgroup per mix (1
-// token 32 us, 10 37, 32 68, 40 80; a workgroup of chains per token: 83).
+// token 29 us, 8 35, 32 64, 40 74; a workgroup of chains per token: 79).
 constexpr int HC_SPLIT_TOKENS = 40;
 
 // Whether the split is the faster, by these fits (us) of what the two do not
@@ -950,8 +953,8 @@ bool split_pays(int K, int mix_n, int n) {
 }
 
 // From this many tokens on they run on the fp32 matrix unit: up to 256 tokens a
-// workgroup of chains per token takes one round of the CUs (85 us; the matrix
-// unit's 82 us and k_hc_finish), 257 take two (164 us against 100).
+// workgroup of chains per token takes one round of the CUs (79 to 82 us; the
+// matrix unit's 83 us and k_hc_finish), 257 take two (160 us against 97).
 constexpr int HC_MFMA_TOKENS = 257;
 constexpr int MX_MAXK = 1 << 20;  // 16 rows and the run-out within a buffer's 32-bit offsets
 

@@ -119,9 +119,9 @@ int dsv4g_gemv_fp8_batch_q(float *y, const float *qx, const float *qscale, int b
                            const uint8_t *W, const uint8_t *S, int in, int out,
                            int round_out, void *stream);
 /* dsv4_gemv_bf16 / _batch (src/dsv4/dsv4_internal.h:256-259); x [batch][in]
- * (16-byte aligned for the streaming kernels), any batch: in runs of 64, 32,
- * 16, 8 or 4 tokens and a remainder of 1-3 when in is a multiple of 64, each
- * run one launch that reads W once. The vocabulary head
+ * (16-byte aligned for the streaming kernels), any batch: in runs of up to 64
+ * tokens when in is a multiple of 64, each run one launch that reads W once.
+ * The vocabulary head
  * (head_logits / head_logits_batch, src/dsv4/dsv4_model.c:7314-7445: the same
  * per-row fmaf chain, logits unrounded) is this call with in = hidden,
  * out = vocab, round_out = 0. */
