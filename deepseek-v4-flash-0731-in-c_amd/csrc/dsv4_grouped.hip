@@ -7,9 +7,9 @@
 //      (the reference's activation quant, exact);
 //   2. router: every logit as the reference's sequential fmaf chain on the
 //      fp32 matrix unit, then the reference's selection and weights - indices
-//      and weights identical to the reference (beyond RX_ALL_TOKENS: BF16 MFMA
-//      logits with sum|g*x| for a rigorous error bound, candidate experts per
-//      token, the chains of the candidates only);
+//      and weights identical to the reference (many tokens of many experts,
+//      router_all: BF16 MFMA logits with sum|g*x| for a rigorous error bound,
+//      candidate experts per token, the chains of the candidates only);
 //   3. dispatch: deterministic per-expert position lists (ascending token, as
 //      expert_forward_batch_routes gathers them, src/dsv4/dsv4_model.c:6498-6524)
 //      and a token-tile table (one workgroup up to 1024 routes); the shared
@@ -162,12 +162,13 @@ __device__ __forceinline__ void rl_mfma(v4f (&acc)[4], v4f (&aab)[4], const RlRe
   }
 }
 
-template <int NS>  // H / 128 when known at compile time (fully unrolled K), else 0
+constexpr int RL_H = 4096;  // hidden: K is fully unrolled
 __global__ __launch_bounds__(256) void k_router_logits_mfma(float *__restrict__ z,
                                                             float *__restrict__ zabs,
                                                             const float *__restrict__ x,
                                                             const uint16_t *__restrict__ G,
-                                                            int T, int H, int E) {
+                                                            int T, int E) {
+  constexpr int H = RL_H, NS = H / 128;
   __shared__ __align__(16) uint16_t xs[2][64 * 136];  // [buf][token][128 + 8 pad] bf16
   const int t0 = blockIdx.x * 64, e0 = blockIdx.y * 64;
   const int tid = threadIdx.x, l = tid % 64;
@@ -193,35 +194,13 @@ __global__ __launch_bounds__(256) void k_router_logits_mfma(float *__restrict__ 
   rl_store(R[0], xs[0], wv, l);
   __syncthreads();
   // step s computes from xs[s & 1] with the gate operands of ring slot s % 3,
-  // stores step s + 1 into the other buffer and loads step s + 2 (loads past
-  // the row end are never used)
-  if constexpr (NS > 0) {
+  // stores step s + 1 into the other buffer and loads step s + 2
 #pragma unroll
-    for (int s = 0; s < NS; ++s) {
-      if (s + 2 < NS) rl_load(R[(s + 2) % 3], rx, xo, xstep, rg, go, 128 * (s + 2));
-      rl_mfma(acc, aab, R[s % 3], xs[s & 1], l);
-      if (s + 1 < NS) {
-        rl_store(R[(s + 1) % 3], xs[(s + 1) & 1], wv, l);
-        __syncthreads();
-      }
-    }
-  } else {
-    // unrolled by three so that the ring slots are compile-time
-    const int ns = H / 128;  // H % 128 == 0
-    for (int s = 0; s < ns; s += 3) {
-      rl_load(R[2], rx, xo, xstep, rg, go, 128 * (s + 2));
-      rl_mfma(acc, aab, R[0], xs[s & 1], l);
-      if (s + 1 < ns) rl_store(R[1], xs[(s + 1) & 1], wv, l);
-      __syncthreads();
-      if (s + 1 >= ns) break;
-      rl_load(R[0], rx, xo, xstep, rg, go, 128 * (s + 3));
-      rl_mfma(acc, aab, R[1], xs[(s + 1) & 1], l);
-      if (s + 2 < ns) rl_store(R[2], xs[s & 1], wv, l);
-      __syncthreads();
-      if (s + 2 >= ns) break;
-      rl_load(R[1], rx, xo, xstep, rg, go, 128 * (s + 4));
-      rl_mfma(acc, aab, R[2], xs[s & 1], l);
-      if (s + 3 < ns) rl_store(R[0], xs[(s + 1) & 1], wv, l);
+  for (int s = 0; s < NS; ++s) {
+    if (s + 2 < NS) rl_load(R[(s + 2) % 3], rx, xo, xstep, rg, go, 128 * (s + 2));
+    rl_mfma(acc, aab, R[s % 3], xs[s & 1], l);
+    if (s + 1 < NS) {
+      rl_store(R[(s + 1) % 3], xs[(s + 1) & 1], wv, l);
       __syncthreads();
     }
   }
@@ -1915,7 +1894,7 @@ namespace {
 struct BatchWs {
   uint16_t *xb, *yb;
   float *z, *zabs, *cscore, *cchoice, *wt, *pos_wt;
-  int *off_bf16, *cand, *ncand, *chain_off;  // with z, zabs: beyond RX_ALL_TOKENS
+  int *off_bf16, *cand, *ncand, *chain_off;  // as z, zabs: unless router_all
   int *rcnt, *idx, *counts, *bh, *pos_off, *tile_off, *pos_token, *pos_route;
   uint16_t *ro;
   size_t bytes;
@@ -1953,15 +1932,24 @@ int side_stream(hipStream_t st, SideStream **out) {
   return 0;
 }
 
-// Up to this many tokens the router's chains run on the VALU (64 tokens 22.8
-// us, 128 27.8, 256 41), beyond on the fp32 matrix unit (38 us from 16 to 256
-// tokens with the GPU to itself).
-#define RX_MAX_TOKENS 192
-// Beyond this many the chains of the candidates only: every expert's chains
-// compete with the shared expert's GEMMs beside them for the matrix unit (layer
-// us, all experts / candidates: 2500 tokens 1478 / 1496, 3000 1656 / 1664, 3500
-// 1825 / 1826, 4096 2035 / 2012, 8192 3577 / 3560).
-#define RX_ALL_TOKENS 3400
+// The router's forms. Every expert's chain on the VALU while that is at most
+// RX_VALU_WGS workgroups (three for each CU; 192 tokens x 256 experts) of at most
+// RX_VALU_TOKENS tokens: 256 experts, 64 tokens 22.8 us, 128 27.8, 256 41, the
+// fp32 matrix unit 38 for 16 to 256 (layer of 193 tokens, 64 experts x 1024: 102 us
+// by the VALU, 108 by the matrix unit). Beyond, on the fp32 matrix unit. Many
+// experts of 4096 columns, whose approximate logits have a fully unrolled kernel,
+// take the candidates' chains only from the size on where every expert's, beside
+// the shared expert's GEMMs, are the slower (layer us, all experts / candidates:
+// 256 experts 2500 tokens 1478 / 1496, 3000 1656 / 1664, 3500 1825 / 1826, 4096 2035 /
+// 2012; by the ratio 512 experts 2000 tokens 1.01, 2800 0.96; 1024 experts 1000
+// 1.03, 2000 0.97; but 128 experts to 16000 tokens 1.04 to 1.01, and at other
+// widths, 1024 to 7168, 256 experts 1.23 to 1.01).
+#define RX_VALU_TOKENS 256
+#define RX_VALU_WGS 768
+// (up to 1024 routes always: k_select_dispatch reads every expert's score)
+bool router_all(int T, int K, int E, int H) {
+  return T * K <= 1024 || H != RL_H || E < 256 || (double)T * T * E <= 2.7e9;  // 256: 3247 tokens
+}
 // Up to this many tokens the shared expert's tiles are folded into the
 // routed GEMM launches (one stream); beyond, they run on a second stream.
 #define FOLD_MAX_TOKENS 256
@@ -1981,7 +1969,7 @@ BatchWs batch_ws_layout(const DSV4GLayer *L, int T, void *base) {
   };
   w.xb = (uint16_t *)take(t * H * 2);
   w.rcnt = (int *)take(4);
-  if (T > RX_ALL_TOKENS) {
+  if (!router_all(T, L->topk, L->n_experts, L->hidden)) {
     w.off_bf16 = (int *)take(t * ((H + 255) / 256) * 4);
     w.z = (float *)take(t * E * 4);
     w.zabs = (float *)take(t * E * 4);
@@ -2047,7 +2035,7 @@ int dsv4g_moe_forward_batch_routes(float *out, const float *x, const DSV4GLayer 
   if (idx_out) w.idx = idx_out;
   if (wt_out) w.wt = wt_out;
 
-  const bool all = T <= RX_ALL_TOKENS;  // every expert's chain
+  const bool all = router_all(T, K, E, H);  // every expert's chain
   // 1. activation quant (+ BF16-valued flags for the candidates' bound)
   {
     const size_t waves = (size_t)T * ((H + 255) / 256);
@@ -2155,22 +2143,17 @@ int dsv4g_moe_forward_batch_routes(float *out, const float *x, const DSV4GLayer 
   if (side) DSV4G_HIP(hipEventRecord(side->join, sst));
   // 2. router: every score exact, or those of the candidates, then the
   // selection (up to 1024 routes it shares a launch with the placement)
-  if (T <= RX_MAX_TOKENS) {
-    hipLaunchKernelGGL(k_router_exact, dim3((unsigned)((T + RX_TOK - 1) / RX_TOK),
-                                            (unsigned)((E + RX_EXP - 1) / RX_EXP)),
-                       dim3(64), 0, st, w.cscore, w.cchoice, x, L->gate_w, L->bias, T, H, E);
+  const int rtok = (T + RX_TOK - 1) / RX_TOK, rexp = (E + RX_EXP - 1) / RX_EXP;
+  if (T <= RX_VALU_TOKENS && (long)rtok * rexp <= RX_VALU_WGS) {
+    hipLaunchKernelGGL(k_router_exact, dim3((unsigned)rtok, (unsigned)rexp), dim3(64), 0, st,
+                       w.cscore, w.cchoice, x, L->gate_w, L->bias, T, H, E);
   } else if (all) {
     DSV4G_TRY(dsv4g_launch_router_scores(w.cscore, w.cchoice, x, L->gate_w, L->bias, T, H, E, st));
   } else {
     const dim3 grid((T + 63) / 64, (E + 63) / 64);
-    if (H == 4096)
-      hipLaunchKernelGGL(k_router_logits_mfma<32>, grid, dim3(256), 0, st, w.z, w.zabs, x,
-                         L->gate_w, T, H, E);
-    else
-      hipLaunchKernelGGL(k_router_logits_mfma<0>, grid, dim3(256), 0, st, w.z, w.zabs, x,
-                         L->gate_w, T, H, E);
-    auto cand = E <= 64 ? k_router_cand<1> : E <= 128 ? k_router_cand<2> : E <= 256 ? k_router_cand<4>
-              : E <= 512 ? k_router_cand<8> : k_router_cand<16>;
+    hipLaunchKernelGGL(k_router_logits_mfma, grid, dim3(256), 0, st, w.z, w.zabs, x, L->gate_w, T,
+                       E);
+    auto cand = E <= 256 ? k_router_cand<4> : E <= 512 ? k_router_cand<8> : k_router_cand<16>;
     hipLaunchKernelGGL(cand, dim3((T + 3) / 4), dim3(256), 0, st, w.cand, w.ncand, w.z, w.zabs,
                        w.off_bf16, (H + 255) / 256, L->bias, L->tid2eid, token_ids, T, H, E, K);
     hipLaunchKernelGGL(k_scan_counts, dim3(1), dim3(1024), 0, st, w.chain_off, w.ncand, T);

@@ -212,13 +212,13 @@ def test_batch_generic_widths(env, hidden, inter, experts, n):
     (1280, 40, 170, 6, 0), (1280, 40, 171, 6, 7), (512, 24, 1024, 1, 0), (512, 24, 1025, 1, 0),
     (384, 16, 600, 3, 5), (128, 5, 192, 2, 0), (128, 5, 193, 2, 0), (384, 320, 901, 6, 0),
     (256, 320, 1700, 6, 0), (128, 320, 2500, 6, 0), (640, 70, 9000, 2, 0),
-    (128, 320, 3400, 6, 0), (128, 320, 3401, 6, 0), (4096, 40, 3450, 6, 0), (640, 70, 4097, 5, 7),
-    (384, 16, 3500, 3, 5), (256, 600, 3407, 8, 0)])
+    (640, 40, 256, 1, 0), (384, 320, 160, 6, 0), (4096, 256, 3247, 6, 0), (4096, 256, 3248, 6, 0),
+    (4096, 300, 3001, 5, 7), (4096, 520, 2290, 3, 0)])
 def test_batch_routing_exact(env, hidden, experts, n, topk, hash_vocab):
-    """The batched router (one lane per chain up to 192 tokens, beyond 16 x 16
-    tiles of chains on the fp32 matrix unit, 1 to 4 token tiles per wave; above
-    3400 tokens the candidates' chains, K below and from 5, hash layers) at
-    ragged token and expert tiles, both forms of the selection (1024 routes and
+    """The batched router (one lane per chain up to 768 workgroups of 8 x 8, beyond
+    16 x 16 tiles of chains on the fp32 matrix unit, 1 to 4 token tiles per wave;
+    very many tokens of 256 or more experts x 4096 the candidates' chains, K below
+    and from 5, hash layers) at ragged token and expert tiles, both forms of the selection (1024 routes and
     more), x not BF16-valued: every route and weight as the oracle's chains and
     selection."""
     orc, lib, dg = env["orc"], env["lib"], env["dg"]
